@@ -1,0 +1,84 @@
+"""Kernels at the sizes where their tiling can go wrong, through the C ABI.
+
+The FP16 gradient is compared with the same network in float64 that rounds the
+activations and the deltas of each layer to FP16, as the kernels store them (a float64
+network without these roundings has other ReLU masks on a few records, which shows when
+there are few records).  What is left is the FP32 order of sums, which moves a rounding
+now and then: 1e-2 in norm holds a few such moves even on one record.
+"""
+import numpy as np
+import pytest
+
+import vknrc_amd as v
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+DEV = "cuda"
+GRAD_F16_TOL = 1e-2
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+def rel_err(y, ref):
+    return float(np.linalg.norm(np.asarray(y, np.float64) - ref) / np.linalg.norm(ref))
+
+
+def gradient_f16(w, hidden, x, t):
+    """d(sum of squared errors)/dw in float64 with FP16 activations and deltas; w, x hold FP16 values."""
+    r16 = lambda a: a.astype(np.float16).astype(np.float64)  # noqa: E731
+    m = [w[4096 * l:4096 * (l + 1)].reshape(64, 64) for l in range(hidden)] + [w[4096 * hidden:].reshape(3, 64)]
+    acts = [x]
+    for l in range(hidden):
+        acts.append(r16(np.maximum(acts[-1] @ m[l].T, 0)))
+    g = r16(2 * (acts[-1] @ m[hidden].T - t))
+    out = []
+    for l in range(hidden, -1, -1):
+        out.append((g.T @ acts[l]).ravel())
+        if l:
+            g = r16((g @ m[l]) * (acts[l] > 0))
+    return np.concatenate(out[::-1])
+
+
+# partial rows of 1, 16, 17, 64, 65 and 256 gradient workgroups: the edges of the three
+# reductions, with full and partial last workgroups; an odd address for the weights
+@pytest.mark.parametrize("hidden", [4, 5])
+@pytest.mark.parametrize("n", [1, 64, 1024, 1025, 4096, 4097, 16384])
+def test_mlp_gradient_reduction_edges(hidden, n):
+    rng = np.random.default_rng(n + hidden)
+    w = rng.normal(0, np.sqrt(2 / 64), v.weight_count(hidden)).astype(np.float16)
+    x = rng.uniform(-1, 1, (n, 64)).astype(np.float16)
+    t = rng.uniform(0, 1, (n, 3)).astype(np.float32)
+    buf = dev(np.concatenate([np.zeros(1, np.float16), w]))
+    dw = torch.full((v.weight_count(hidden),), 7.0, device=DEV)
+    v.mlp_gradient_f16(buf[1:], dev(x), dev(t), n, dw, hidden_layers=hidden)
+    G = gradient_f16(w.astype(np.float64), hidden, x.astype(np.float64), t.astype(np.float64))
+    assert rel_err(host(dw), G) < GRAD_F16_TOL
+
+
+# the forward gathers row-major weights with wide loads where their address allows it and
+# single halves where it does not: the same fragments, so the same bits
+@pytest.mark.parametrize("hidden", [4, 5])
+@pytest.mark.parametrize("n", [1, 63, 65, 4097])
+def test_mlp_forward_weight_alignment(hidden, n):
+    rng = np.random.default_rng(n + hidden)
+    w = rng.normal(0, np.sqrt(2 / 64), v.weight_count(hidden)).astype(np.float16)
+    x = dev(rng.uniform(-1, 1, (n, 64)).astype(np.float16))
+    out = []
+    for shift in (0, 1, 2, 4):
+        buf = dev(np.concatenate([np.zeros(shift, np.float16), w]))
+        out.append(torch.full((n, 3), 7.0, device=DEV))
+        v.mlp_forward_f16(buf[shift:], x, n, out[-1], hidden_layers=hidden)
+    m = [w.astype(np.float64)[4096 * l:4096 * (l + 1)].reshape(64, 64) for l in range(hidden)]
+    a = host(x).astype(np.float64)
+    for l in range(hidden):
+        a = np.maximum(a @ m[l].T, 0).astype(np.float16).astype(np.float64)
+    assert rel_err(host(out[0]), a @ w.astype(np.float64)[4096 * hidden:].reshape(3, 64).T) < GRAD_F16_TOL
+    assert all(torch.equal(o, out[0]) for o in out)

@@ -259,6 +259,86 @@ nrc_status check_train(nrc_cache *c, const nrc_train_record *d_records, uint32_t
 }
 
 
+// Scratch of the stateless gradient (nrc_mlp_gradient_f16): a few blocks per GPU kept
+// between calls, each guarded by the event of its last use.  A call takes a block that no
+// other host thread holds, makes its stream wait for that event (on whatever stream it was
+// recorded) and records the event again after its last kernel, so calls on several streams
+// and threads never share a block in use.  With no block free, or under stream capture,
+// the scratch is stream-ordered as a library's is (hipMallocAsync, hipFreeAsync).  Those
+// two cost 25-40 us of host time a call: a forward and a gradient of 16,384 rows took
+// 109 us a pass with them, 33 us of it in kernels (38 us a pass with a kept block).
+constexpr int kMaxDevices = 64, kScratchBlocks = 2;
+// one gradient workgroup a CU writes one row: 256 rows and both fragment copies, 21.3 MB
+constexpr size_t kScratchBytes = 2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDEN_LAYERS) + nrc::bwd_frag_halves(NRC_MAX_HIDDEN_LAYERS)) +
+                                 sizeof(float) * (((size_t)nrc::weight_count(NRC_MAX_HIDDEN_LAYERS) + 64) & ~size_t(63)) * 256;
+struct ScratchBlock {
+	void *p = nullptr;
+	hipEvent_t done = nullptr;
+	bool held = false;
+};
+std::mutex g_scratch_mu;
+ScratchBlock g_scratch[kMaxDevices][kScratchBlocks];
+
+struct Scratch {
+	void *p = nullptr;
+	ScratchBlock *block = nullptr; // null: stream-ordered
+
+	hipError_t take(size_t bytes, hipStream_t s) {
+		int dev = 0;
+		hipError_t e = hipGetDevice(&dev);
+		if (e != hipSuccess) return e;
+		hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+		const bool captured = hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+		if (!captured && bytes <= kScratchBytes && dev >= 0 && dev < kMaxDevices) {
+			std::lock_guard<std::mutex> lock(g_scratch_mu);
+			for (ScratchBlock &b : g_scratch[dev]) {
+				if (b.held) continue;
+				if (!b.p) {
+					hipEvent_t done = nullptr;
+					void *q = nullptr;
+					if (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) break;
+					if (hipMalloc(&q, kScratchBytes) != hipSuccess) {
+						(void)hipEventDestroy(done);
+						break;
+					}
+					b.p = q;
+					b.done = done;
+				} else if (hipStreamWaitEvent(s, b.done, 0) != hipSuccess) {
+					break;
+				}
+				b.held = true;
+				block = &b;
+				p = b.p;
+				return hipSuccess;
+			}
+		}
+		(void)hipGetLastError();
+		return hipMallocAsync(&p, bytes, s);
+	}
+
+	// after the last kernel that uses the scratch was launched, whatever failed
+	hipError_t give(hipStream_t s) {
+		if (!block) return hipFreeAsync(p, s);
+		std::lock_guard<std::mutex> lock(g_scratch_mu);
+		const hipError_t e = hipEventRecord(block->done, s);
+		if (e == hipSuccess) block->held = false; // a block whose use cannot be marked is never handed out again
+		return e;
+	}
+};
+
+// Frees the kept blocks of this GPU that no call holds (hipFree waits for their last use).
+void trim_scratch() {
+	int dev = 0;
+	if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return;
+	std::lock_guard<std::mutex> lock(g_scratch_mu);
+	for (ScratchBlock &b : g_scratch[dev])
+		if (b.p && !b.held) {
+			(void)hipFree(b.p);
+			(void)hipEventDestroy(b.done);
+			b = ScratchBlock{};
+		}
+}
+
 // One training step on stream s (arguments already checked).
 nrc_status train_step(nrc_cache *c, const nrc_train_record *d_records, const uint32_t *d_count, uint32_t max_count,
                       nrc_path path, uint32_t flags, hipStream_t s) {
@@ -395,18 +475,26 @@ nrc_status nrc_cache_create(const nrc_cache_desc *desc, nrc_cache **out) {
 	c->part_cap = (desc->train_batch_size + nrc::kFusedSmallRecords - 1) / nrc::kFusedSmallRecords;
 	const CacheSizes sz(*desc);
 	hipError_t e = hipGetDevice(&c->device);
-	if (e == hipSuccess) e = hipMalloc(&c->entries, sz.entries);
-	if (e == hipSuccess) e = hipMalloc(&c->w16, sz.w16);
-	if (e == hipSuccess) e = hipMalloc(&c->wf, sz.wf);
-	if (e == hipSuccess) e = hipMalloc(&c->wtf, sz.wtf);
-	if (e == hipSuccess) e = hipMalloc(&c->usef, sz.usef);
-	if (e == hipSuccess) e = hipMalloc(&c->w8, sz.w8);
-	if (e == hipSuccess) e = hipMalloc(&c->f8, sz.f8);
-	if (e == hipSuccess) e = hipMalloc(&c->use16, sz.use16);
-	if (e == hipSuccess) e = hipMalloc(&c->w32, sz.w32);
-	if (e == hipSuccess) e = hipMalloc(&c->use32, sz.use32);
-	if (e == hipSuccess) e = hipMalloc(&c->state, sz.state);
-	if (e == hipSuccess) e = hipMalloc(&c->partials, sz.partials);
+	auto alloc = [&](auto **p, size_t bytes) {
+		if (e != hipSuccess) return;
+		e = hipMalloc(p, bytes);
+		if (e != hipErrorOutOfMemory) return;
+		trim_scratch(); // kept scratch goes before a cache is refused
+		(void)hipGetLastError();
+		e = hipMalloc(p, bytes);
+	};
+	alloc(&c->entries, sz.entries);
+	alloc(&c->w16, sz.w16);
+	alloc(&c->wf, sz.wf);
+	alloc(&c->wtf, sz.wtf);
+	alloc(&c->usef, sz.usef);
+	alloc(&c->w8, sz.w8);
+	alloc(&c->f8, sz.f8);
+	alloc(&c->use16, sz.use16);
+	alloc(&c->w32, sz.w32);
+	alloc(&c->use32, sz.use32);
+	alloc(&c->state, sz.state);
+	alloc(&c->partials, sz.partials);
 
 	if (e != hipSuccess) {
 		free_cache(c);
@@ -730,17 +818,9 @@ nrc_status nrc_mlp_forward_f16(uint32_t hidden, const uint16_t *d_w, const uint1
 	if (!d_w || !d_in || !d_out) return fail(NRC_ERROR_INVALID_ARGUMENT, "NULL buffer");
 	if (check_count(n) != NRC_OK) return NRC_ERROR_CAPACITY;
 	const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-	const size_t nf = nrc::fwd_frag_halves((int)hidden);
-	_Float16 *wf = nullptr;
-	NRC_HIP(hipMallocAsync(reinterpret_cast<void **>(&wf), 2 * nf, s), "forward scratch");
-	hipError_t e = hipMemsetAsync(wf, 0, 2 * nf, s);
-	if (e == hipSuccess)
-		e = nrc::launch_make_frags((int)hidden, reinterpret_cast<const _Float16 *>(d_w), wf, nullptr, s);
-	if (e == hipSuccess)
-		e = nrc::launch_fused_forward_f16((int)hidden, reinterpret_cast<const _Float16 *>(d_in), n, wf, d_out, s);
-	hipError_t e2 = hipFreeAsync(wf, s);
+	const hipError_t e = nrc::launch_fused_forward_f16((int)hidden, reinterpret_cast<const _Float16 *>(d_in), n,
+	                                                   reinterpret_cast<const _Float16 *>(d_w), d_out, s);
 	if (e != hipSuccess) return hip_fail(e, "nrc_mlp_forward_f16");
-	if (e2 != hipSuccess) return hip_fail(e2, "nrc_mlp_forward_f16 free");
 	return NRC_OK;
 }
 
@@ -752,32 +832,22 @@ nrc_status nrc_mlp_gradient_f16(uint32_t hidden, const uint16_t *d_w, const uint
 	const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 	const uint32_t wc = nrc_weight_count(hidden);
 	const uint32_t pstride = ((wc + 1) + 63u) & ~63u;
-	// enough partial rows for any plan: one per 64 records
-	const uint32_t nb = n == 0 ? 1 : (n + nrc::kFusedSmallRecords - 1) / nrc::kFusedSmallRecords;
+	const uint32_t nb = nrc::plan_fused_gradient(n).blocks; // partial rows
 	const size_t nf = nrc::fwd_frag_halves((int)hidden), nt = nrc::bwd_frag_halves((int)hidden);
-	float *partials = nullptr;
-	_Float16 *wf = nullptr, *wtf = nullptr;
-	hipError_t e = hipMallocAsync(reinterpret_cast<void **>(&partials), sizeof(float) * (size_t)pstride * nb, s);
-	if (e == hipSuccess) e = hipMallocAsync(reinterpret_cast<void **>(&wf), 2 * nf, s);
-	if (e == hipSuccess) e = hipMallocAsync(reinterpret_cast<void **>(&wtf), 2 * nt, s);
+	// the forward and the backward fragments and the partial rows
+	Scratch scr;
+	NRC_HIP(scr.take(2 * (nf + nt) + sizeof(float) * (size_t)pstride * nb, s), "gradient scratch");
+	_Float16 *wf = static_cast<_Float16 *>(scr.p), *wtf = wf + nf;
+	float *partials = reinterpret_cast<float *>(wtf + nt);
 	uint32_t nparts = 0;
-	const _Float16 *w = reinterpret_cast<const _Float16 *>(d_w);
-	if (e == hipSuccess) e = hipMemsetAsync(wf, 0, 2 * nf, s);
-	if (e == hipSuccess) e = hipMemsetAsync(wtf, 0, 2 * nt, s);
-	if (e == hipSuccess) e = nrc::launch_make_frags((int)hidden, w, wf, wtf, s);
+	hipError_t e = nrc::launch_make_frags((int)hidden, reinterpret_cast<const _Float16 *>(d_w), wf, wtf, s);
 	if (e == hipSuccess)
 		e = nrc::launch_fused_gradient_f16((int)hidden, reinterpret_cast<const _Float16 *>(d_in), d_targets, n, wf, wtf,
 		                                   partials, pstride, &nparts, s);
 	if (e == hipSuccess) e = nrc::launch_reduce_partials(partials, nparts, pstride, wc, d_dw, s);
-	// every scratch buffer that was allocated is freed, whatever failed
-	hipError_t e2 = hipSuccess;
-	for (void *p : {static_cast<void *>(partials), static_cast<void *>(wf), static_cast<void *>(wtf)})
-		if (p) {
-			const hipError_t f = hipFreeAsync(p, s);
-			if (e2 == hipSuccess) e2 = f;
-		}
+	const hipError_t e2 = scr.give(s); // whatever failed
 	if (e != hipSuccess) return hip_fail(e, "nrc_mlp_gradient_f16");
-	if (e2 != hipSuccess) return hip_fail(e2, "nrc_mlp_gradient_f16 free");
+	if (e2 != hipSuccess) return hip_fail(e2, "nrc_mlp_gradient_f16 scratch");
 	return NRC_OK;
 }
 
@@ -840,14 +910,10 @@ nrc_status nrc_mlp_gradient_f16_noalloc(uint32_t hidden, const uint16_t *d_w, co
 	const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 	const uint32_t wc = nrc_weight_count(hidden);
 	const uint32_t pstride = ((wc + 1) + 63u) & ~63u;
-	const size_t nf = nrc::fwd_frag_halves((int)hidden), nt = nrc::bwd_frag_halves((int)hidden);
 	_Float16 *wf = reinterpret_cast<_Float16 *>(base);
 	_Float16 *wtf = reinterpret_cast<_Float16 *>(base + kNoallocWfBytes);
 	float *partials = reinterpret_cast<float *>(base + kNoallocWfBytes + kNoallocWtfBytes);
-	// the fragment copies keep the last call's values: their padding must start at zero
-	hipError_t e = nrc::launch_zero_words(reinterpret_cast<uint32_t *>(wf), nf / 2, s);
-	if (e == hipSuccess) e = nrc::launch_zero_words(reinterpret_cast<uint32_t *>(wtf), nt / 2, s);
-	if (e == hipSuccess) e = nrc::launch_make_frags((int)hidden, reinterpret_cast<const _Float16 *>(d_w), wf, wtf, s);
+	hipError_t e = nrc::launch_make_frags((int)hidden, reinterpret_cast<const _Float16 *>(d_w), wf, wtf, s);
 	uint32_t nparts = 0;
 	if (e == hipSuccess)
 		e = nrc::launch_fused_gradient_f16((int)hidden, reinterpret_cast<const _Float16 *>(d_in), d_targets, n, wf, wtf,

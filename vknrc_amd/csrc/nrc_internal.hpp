@@ -39,7 +39,7 @@ struct InferItem {
 	const float *queries;    // [max_count][14]
 	const uint32_t *d_count; // device count or null (= max_count)
 	float *out;              // [max_count][3]
-	const _Float16 *wf;      // fragment-major use-weights (FP16 path)
+	const _Float16 *wf;      // fragment-major use-weights (FP16 path); row-major with fin
 	const uint8_t *w8;       // fragment-major fp8 use-weights (FP8 path)
 	Fp8State *f8;            // FP8 path: scales in, activation maxima out
 	uint32_t max_count;
@@ -156,12 +156,8 @@ hipError_t launch_adam_group(AdamGroup &grp, hipStream_t stream);
 hipError_t launch_reduce_partials(const float *partials, uint32_t nparts, uint32_t pstride, uint32_t n, float *out,
                                   hipStream_t stream);
 hipError_t launch_init_state(DeviceState *st, float loss_scale, hipStream_t stream);
-// Scatters row-major fp16 weights into the fragment-major copies (whose padding
-// must already be zero); wtf may be null.
+// Writes the fragment-major copies of row-major fp16 weights, padding included; wtf may be null.
 hipError_t launch_make_frags(int hidden, const _Float16 *w16, _Float16 *wf, _Float16 *wtf, hipStream_t stream);
-// Zeroes `words` 32-bit words at dst with a kernel (no memset node, so the launch
-// may be captured into a graph).
-hipError_t launch_zero_words(uint32_t *dst, size_t words, hipStream_t stream);
 
 // nrc_records.hip: the record front-end, the wire-record epilogue, the path
 // suffix sums and the screen pass
@@ -188,8 +184,8 @@ hipError_t launch_fused_infer_group(int hidden, int encoding, InferGroup &grp, h
 // use32; then the grouped FP8 inference.
 hipError_t launch_fp8_infer_group(int hidden, int encoding, InferGroup &grp, const float *const *use32,
                                   uint8_t *const *w8, hipStream_t stream);
-// Forward over n pre-encoded fp16 input rows with fragment-major weights wf (no clamp).
-hipError_t launch_fused_forward_f16(int hidden, const _Float16 *inputs, uint32_t n, const _Float16 *wf, float *out,
+// Forward over n pre-encoded fp16 input rows with row-major fp16 weights (no clamp).
+hipError_t launch_fused_forward_f16(int hidden, const _Float16 *inputs, uint32_t n, const _Float16 *w16, float *out,
                                     hipStream_t stream);
 // Workgroups and chunking of the fused gradient for a step of n records: chunks
 // 64-record chunks a workgroup (0: from n and the CU count).  The chunking fixes

@@ -195,26 +195,76 @@ template <int U, int W> __global__ __launch_bounds__(256) void adam_kernel(const
 	}
 }
 
-// out[i] = sum_q partials[q][i] in a fixed order (the gradient-only entry point).
+// out[i] = sum_q partials[q][i] in a fixed order (the gradient-only entry point): 64
+// weights a block, 16 threads a row (float4 each), 16 rows a pass and U passes in
+// flight, as adam_kernel sums them.  Bound by the latency and bandwidth of the rows
+// (21 MB for 16,384 records); one thread a weight walking the rows one after another
+// took 91 us for 256 rows (a serial chain of loads in 81 blocks), this takes 5.8 us.
+template <int U>
 __global__ __launch_bounds__(256) void reduce_kernel(const float *__restrict__ partials, uint32_t nparts,
-                                                     uint32_t pstride, uint32_t n, float *__restrict__ out) {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
-	float s = 0.0f;
-	for (uint32_t q = 0; q < nparts; ++q) s += partials[(size_t)q * pstride + i];
-	out[i] = s;
+                                                     uint32_t pstride, float *__restrict__ out) {
+	const int t = threadIdx.x, col4 = t & 15, slice = t >> 4;
+	const uint32_t w0 = blockIdx.x * 64u, lastrow = nparts - 1;
+	const f4v *src = reinterpret_cast<const f4v *>(partials + w0) + col4;
+	const size_t ps4 = pstride / 4;
+	float4 acc[U];
+#pragma unroll
+	for (int u = 0; u < U; ++u) acc[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	for (uint32_t q = slice; q < nparts; q += 16 * U) {
+		f4v x[U];
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			const uint32_t row = q + 16 * u;
+			x[u] = __builtin_nontemporal_load(src + (size_t)(row < lastrow ? row : lastrow) * ps4);
+		}
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			const bool in = q + 16 * u < nparts;
+			acc[u].x += in ? x[u][0] : 0.0f;
+			acc[u].y += in ? x[u][1] : 0.0f;
+			acc[u].z += in ? x[u][2] : 0.0f;
+			acc[u].w += in ? x[u][3] : 0.0f;
+		}
+	}
+#pragma unroll
+	for (int u = 1; u < U; ++u) {
+		acc[0].x += acc[u].x; acc[0].y += acc[u].y; acc[0].z += acc[u].z; acc[0].w += acc[u].w;
+	}
+	__shared__ float4 red[16][16];
+	red[slice][col4] = acc[0];
+	__syncthreads();
+	if (t < 64) {
+		const float *rf = reinterpret_cast<const float *>(&red[0][0]);
+		float g = 0.0f;
+#pragma unroll
+		for (int sl = 0; sl < 16; ++sl) g += rf[sl * 64 + t];
+		out[w0 + t] = g;
+	}
 }
 
+// The fragment-major copies of row-major fp16 weights, one 8-half fragment of one lane
+// a thread, padding included: the gather writes every half of both copies, so neither
+// needs clearing first (two fills and a scatter before).  The weights are read as
+// single halves, which any alignment of the caller's buffer allows.
 __global__ __launch_bounds__(256) void make_frags_kernel(const _Float16 *__restrict__ w16, _Float16 *__restrict__ wf,
-                                                         _Float16 *__restrict__ wtf, uint32_t n) {
-	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n) return;
-	frag_scatter(i, w16[i], wf, wtf);
-}
-
-__global__ __launch_bounds__(256) void zero_words_kernel(uint32_t *__restrict__ dst, size_t words) {
-	for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (size_t)gridDim.x * blockDim.x)
-		dst[i] = 0u;
+                                                         _Float16 *__restrict__ wtf, int hidden) {
+	typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+	const int nf = (int)fwd_frag_halves(hidden) / 8, nt = wtf ? (int)bwd_frag_halves(hidden) / 8 : 0;
+	const int f = (int)(blockIdx.x * 256u + threadIdx.x);
+	if (f >= nf + nt) return;
+	const bool bwd = f >= nf;
+	const int k = bwd ? f - nf : f;
+	// block = 8 * layer slot + 2 * mt + c; lane 16 g + r holds row 16 mt + r at 8 columns
+	const int slot = k >> 9, row = 16 * ((k >> 7) & 3) + (k & 15), c = (k >> 6) & 1, g = (k >> 4) & 3;
+	const int layer = bwd ? slot + 1 : slot;
+	h8 h;
+#pragma unroll
+	for (int j = 0; j < 8; ++j) {
+		const int col = 32 * c + 4 * g + (j < 4 ? j : 12 + j);
+		const int out = bwd ? col : row, in = bwd ? row : col; // W_layer[out][in]
+		h[j] = (layer < hidden || out < kOut) ? w16[(layer * kWidth + out) * kWidth + in] : (_Float16)0.0f;
+	}
+	*reinterpret_cast<h8 *>((bwd ? wtf : wf) + (size_t)k * 8) = h;
 }
 
 __global__ void init_state_kernel(DeviceState *st, float loss_scale) {
@@ -269,21 +319,16 @@ hipError_t launch_adam(const AdamArgs &a, hipStream_t stream) {
 
 hipError_t launch_reduce_partials(const float *partials, uint32_t nparts, uint32_t pstride, uint32_t n, float *out,
                                   hipStream_t stream) {
-	reduce_kernel<<<dim3((n + 255) / 256), dim3(256), 0, stream>>>(partials, nparts, pstride, n, out);
+	const dim3 g(n / 64), b(256); // weight counts are multiples of 64
+	if (nparts <= 16) reduce_kernel<1><<<g, b, 0, stream>>>(partials, nparts, pstride, out);
+	else if (nparts <= 64) reduce_kernel<4><<<g, b, 0, stream>>>(partials, nparts, pstride, out);
+	else reduce_kernel<16><<<g, b, 0, stream>>>(partials, nparts, pstride, out);
 	return hipGetLastError();
 }
 
 hipError_t launch_make_frags(int hidden, const _Float16 *w16, _Float16 *wf, _Float16 *wtf, hipStream_t stream) {
-	const uint32_t n = (uint32_t)weight_count(hidden);
-	make_frags_kernel<<<dim3((n + 255) / 256), dim3(256), 0, stream>>>(w16, wf, wtf, n);
-	return hipGetLastError();
-}
-
-hipError_t launch_zero_words(uint32_t *dst, size_t words, hipStream_t stream) {
-	if (words == 0) return hipSuccess;
-	size_t blocks = (words + 255) / 256;
-	if (blocks > 1024) blocks = 1024;
-	zero_words_kernel<<<dim3((uint32_t)blocks), dim3(256), 0, stream>>>(dst, words);
+	const uint32_t n = (fwd_frag_halves(hidden) + (wtf ? bwd_frag_halves(hidden) : 0u)) / 8u;
+	make_frags_kernel<<<dim3((n + 255) / 256), dim3(256), 0, stream>>>(w16, wf, wtf, hidden);
 	return hipGetLastError();
 }
 
