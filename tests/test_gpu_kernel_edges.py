@@ -10,6 +10,8 @@ import numpy as np
 import pytest
 
 import vknrc_amd as v
+from oracle.oracle import Oracle
+from vknrc_amd import workloads as wl
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +84,52 @@ def test_mlp_forward_weight_alignment(hidden, n):
         a = np.maximum(a @ m[l].T, 0).astype(np.float16).astype(np.float64)
     assert rel_err(host(out[0]), a @ w.astype(np.float64)[4096 * hidden:].reshape(3, 64).T) < GRAD_F16_TOL
     assert all(torch.equal(o, out[0]) for o in out)
+
+
+# FP32 sums of 64 products over at most 6 layers are within 6 * 64 * 2^-24 = 2.3e-5 of their
+# exact values relative to the largest terms; the gradient passes through three such chains.
+PLAIN_TOL, PLAIN_GRAD_TOL = 2.3e-5, 7e-5
+ENCODINGS = [(5, v.ENCODING_TRI12), (5, v.ENCODING_SINCOS6), (4, v.ENCODING_UV_SINCOS16)]
+
+
+def plain_inputs(hidden, enc, n):
+    rng = np.random.default_rng(100 * n + hidden + enc)
+    r = wl.make_train_records(n, rng, wl.GaussianLights(7))
+    if enc == v.ENCODING_UV_SINCOS16:
+        r[:, :2] = rng.uniform(0, 1, (n, 2))
+    return rng.normal(0, np.sqrt(2 / 64), v.weight_count(hidden)).astype(np.float32), r
+
+
+# 16-record tiles over one workgroup a CU: partial tiles, one tile more than CUs, waves with
+# no tile, and a device count that ends inside a tile
+@pytest.mark.parametrize("hidden,enc", ENCODINGS)
+@pytest.mark.parametrize("n,live", [(1, 1), (16, 16), (17, 17), (4112, 4097), (33000, 32769)])
+def test_plain_inference_tiles(hidden, enc, n, live):
+    w, r = plain_inputs(hidden, enc, n)
+    st = v.NRCState(v.NRCConfig(hidden_layers=hidden, encoding=enc))
+    st.set_state(weight=w)
+    out = torch.full((n, 3), 7.0, device=DEV)
+    st.infer(dev(r[:, :14]), out, count=dev(np.array([live], np.uint32).view(np.int32)), path=v.PATH_PLAIN_F32)
+    y = host(out)
+    f = Oracle("f32").encode(r[:live], enc).astype(np.float64)  # features rounded as FP32 computes them
+    ref = np.maximum(Oracle("f64").infer_encoded(w.astype(np.float64), hidden, f), 0)
+    assert rel_err(y[:live], ref) < PLAIN_TOL
+    assert (y[live:] == 7.0).all()
+    st.close()
+
+
+# the chunks of the FP32 weight gradient: inside one tile, at its edges, at the edges of a
+# 256-record chunk, many chunks with a partial last one, and a device count below the size
+@pytest.mark.parametrize("hidden,enc", ENCODINGS)
+@pytest.mark.parametrize("n,live", [(1, 1), (16, 16), (17, 17), (256, 256), (257, 257), (8193, 8100)])
+def test_plain_gradient_chunks(hidden, enc, n, live):
+    w, r = plain_inputs(hidden, enc, n)
+    st = v.NRCState(v.NRCConfig(hidden_layers=hidden, encoding=enc, loss=v.LOSS_L2))
+    st.set_state(weight=w)
+    st.train(dev(r), count=dev(np.array([live], np.uint32).view(np.int32)), path=v.PATH_PLAIN_F32)
+    s = st.get_state()
+    f = Oracle("f32").encode(r[:live], enc).astype(np.float64)
+    G, loss = Oracle("f64").gradient_encoded(w.astype(np.float64), hidden, f, r[:live, 14:].astype(np.float64), loss=1)
+    assert rel_err(s["m"] / (1.0 - np.float32(0.9)), G / live) < PLAIN_GRAD_TOL
+    assert abs(s["state"]["last_loss"] / (loss / live) - 1) < PLAIN_GRAD_TOL
+    st.close()

@@ -471,7 +471,7 @@ nrc_status nrc_cache_create(const nrc_cache_desc *desc, nrc_cache **out) {
 	c->desc = *desc;
 	c->wc = nrc_weight_count(desc->hidden_layers);
 	c->pstride = ((c->wc + 1) + 63u) & ~63u;
-	// one partial row per 64 records covers every fused-gradient plan (and the plain path's 512)
+	// one partial row per 64 records covers every fused-gradient plan (and the plain path)
 	c->part_cap = (desc->train_batch_size + nrc::kFusedSmallRecords - 1) / nrc::kFusedSmallRecords;
 	const CacheSizes sz(*desc);
 	hipError_t e = hipGetDevice(&c->device);

@@ -102,7 +102,7 @@ struct TrainArgs {
 	int parity;      // state buffer this step reads
 	float *partials; // [nparts][pstride]
 	uint32_t pstride;
-	// plain-path scratch, feature-major [(hidden+1)][64][ldn]
+	// plain-path scratch, [hidden + 1][ldn / 16 tiles][64 features][16 records]
 	float *acts, *deltas, *sample_loss;
 	uint32_t ldn;
 };

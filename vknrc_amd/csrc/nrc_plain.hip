@@ -1,80 +1,155 @@
-// nrc_plain.hip -- the plain method: FP32 encoding, weights and accumulation.
+// nrc_plain.hip -- the plain method: FP32 encoding, weights, products and sums.
 //
-// One thread per record, all weights of the network staged in LDS as FP32, the
-// 64-wide activation vector held in VGPRs.  The weight gradient is reduced over
-// fixed 512-record chunks in a fixed order, so the result is deterministic.
-// This path is the FP32 reference the fused FP16-MFMA path is measured against.
+// The layers run on v_mfma_f32_16x16x4_f32, whose products and sums are FP32: twice the
+// rate of FP32 FMAs without packed instructions.  Lane l = 16 g + r holds A row r, B
+// column r at K index g, and D column r, rows 4 g .. 4 g + 3.  A wave runs 16 records
+// (the columns).  The rows of an A tile are permuted so that D element i of tile Mt in
+// lane group g is unit 16 Mt + 4 i + g: K step s = 4 mt + i of the next layer takes
+// features 4 s .. 4 s + 3 from lane groups 0 .. 3, which is exactly where they are.  So a
+// layer's ReLU'd D registers are the next layer's B operands with no data movement at
+// all, and every sum runs over k = 0 .. 63 in order, one fused multiply-add after the
+// other, as one thread a record would compute it (the MFMA adds its K products in order,
+// each rounded: the results equal the FMA loop's bit for bit).
+//
+// All weights of the network lie in LDS as A fragments: float4 (l, Mt, mt, g, r) holds
+// W_l[16 Mt + 4 (r & 3) + (r >> 2)][16 mt + 4 i + g], i = 0..3, at slot 16 g + ((r + g) & 15)
+// of its 1 KB block.  The rotation by g lets the backward read single floats of W_l^T from
+// the same copy without bank conflicts (for one i, the 16 values (4 g + i + g') mod 16 of
+// g, g' in 0..3 differ).
+//
+// The weight gradient is reduced over fixed kPlainChunk-record chunks in a fixed order,
+// so the result is deterministic.  This path is the FP32 reference the fused FP16-MFMA
+// path is measured against.
+#include <type_traits>
+
 #include "nrc_internal.hpp"
 
 namespace nrc {
 
 namespace {
 
-// Output units between scheduling barriers in the FP32 forward: groups of 4
-// keep the H = 5 kernel within 256 VGPRs without spilling.
-constexpr int kPlainSchedGroup = 4;
+typedef float float4_t __attribute__((ext_vector_type(4)));
 
-// x (64 input features) -> a_H in x, returns the 3 raw outputs in o.
-// a_{l+1} = relu(W_l a_l) (NN_nv.glsl:99-127), o = W_H a_H (NN_nv.glsl:129-158).
-template <int H> __device__ __forceinline__ void forward_f32(const float *sW, float *x, float *o) {
-#pragma unroll 1
-	for (int l = 0; l < H; ++l) {
-		const float *Wl = sW + l * kWidth * kWidth;
-		float y[kWidth];
+constexpr int kPlainWaves = 8; // waves of a workgroup; one workgroup a CU (its LDS holds the FP32 weights)
+
+__device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) {
+	return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int H> struct PlainSmem {
+	float4_t frag[H * 16 * 64];
+	float4_t frag_out[4 * 64]; // the output layer's A fragments: row c < 3 is output c, the rest zero
+};
+
+// All weights into LDS, every load in flight before the first store.
+template <int H> __device__ __forceinline__ void stage_weights(PlainSmem<H> &S, const float *__restrict__ w32) {
+	constexpr int kPer = H * 1024 / (64 * kPlainWaves);
+	const int t = threadIdx.x;
+	const float4_t *src = reinterpret_cast<const float4_t *>(w32);
+	float4_t v[kPer];
 #pragma unroll
-		for (int m = 0; m < kWidth; ++m) {
-			float acc = 0.0f;
-#pragma unroll
-			for (int k = 0; k < kWidth; k += 4) {
-				const float4 w = *reinterpret_cast<const float4 *>(Wl + m * kWidth + k);
-				acc = fmaf(w.x, x[k + 0], acc);
-				acc = fmaf(w.y, x[k + 1], acc);
-				acc = fmaf(w.z, x[k + 2], acc);
-				acc = fmaf(w.w, x[k + 3], acc);
-			}
-			y[m] = fmaxf(acc, 0.0f);
-			// bound how far the weight loads run ahead (and the registers they hold)
-			if (m % kPlainSchedGroup == kPlainSchedGroup - 1) __builtin_amdgcn_sched_barrier(0);
-		}
-#pragma unroll
-		for (int m = 0; m < kWidth; ++m) x[m] = y[m];
+	for (int k = 0; k < kPer; ++k) v[k] = src[t + k * 64 * kPlainWaves];
+	if (t < 4 * 64) {
+		const int mt = t >> 6, g = (t >> 4) & 3, r = t & 15;
+		const float *wo = w32 + H * kWidth * kWidth + (r < kOut ? r : 0) * kWidth + 16 * mt + g;
+		const float4_t o = {wo[0], wo[4], wo[8], wo[12]};
+		S.frag_out[t] = r < kOut ? o : (float4_t)0.0f;
 	}
-	const float *Wo = sW + H * kWidth * kWidth;
+	float *f = reinterpret_cast<float *>(S.frag);
 #pragma unroll
-	for (int c = 0; c < kOut; ++c) {
-		float acc = 0.0f;
+	for (int k = 0; k < kPer; ++k) {
+		// layer j >> 10, row (j >> 4) & 63, columns 16 mt + 4 i + 0..3
+		const int j = t + k * 64 * kPlainWaves, row = (j >> 4) & 63, mt = (j >> 2) & 3, i = j & 3;
+		const int r = 4 * (row & 3) + ((row >> 2) & 3), blk = ((j >> 10) * 4 + (row >> 4)) * 4 + mt;
 #pragma unroll
-		for (int k = 0; k < kWidth; k += 4) {
-			const float4 w = *reinterpret_cast<const float4 *>(Wo + c * kWidth + k);
-			acc = fmaf(w.x, x[k + 0], acc);
-			acc = fmaf(w.y, x[k + 1], acc);
-			acc = fmaf(w.z, x[k + 2], acc);
-			acc = fmaf(w.w, x[k + 3], acc);
+		for (int g = 0; g < 4; ++g) f[(blk * 64 + 16 * g + ((r + g) & 15)) * 4 + i] = v[k][g];
+	}
+	__syncthreads();
+}
+
+__device__ __forceinline__ float4_t relu4(float4_t v) {
+#pragma unroll
+	for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.0f);
+	return v;
+}
+
+// The features 4 s + g, s = 0..15, of one record for lane group g (element g of every
+// quad), by the arithmetic of encode_all.
+template <int ENC> __device__ __forceinline__ void encode_lane(const float *rec, int g, float4_t *x) {
+	auto pick = [g](float a, float b, float c, float d) __attribute__((always_inline)) {
+		return g == 0 ? a : g == 1 ? b : g == 2 ? c : d;
+	};
+	if constexpr (ENC == NRC_ENCODING_UV_SINCOS16) {
+#pragma unroll
+		for (int a = 0; a < 2; ++a)
+#pragma unroll
+			for (int q = 0; q < 4; ++q) {
+				float s[4], c[4];
+				sincospi_poly(rec[a] * (float)(1 << (4 * q)), &s[0], &c[0]);
+#pragma unroll
+				for (int k = 1; k < 4; ++k) {
+					s[k] = 2.0f * s[k - 1] * c[k - 1];
+					c[k] = 1.0f - 2.0f * s[k - 1] * s[k - 1];
+				}
+				x[2 * a][q] = pick(s[0], s[1], s[2], s[3]);
+				x[2 * a + 1][q] = pick(c[0], c[1], c[2], c[3]);
+			}
+	} else {
+#pragma unroll
+		for (int a = 0; a < 3; ++a) {
+			if constexpr (ENC == NRC_ENCODING_TRI12) {
+				const float p = rec[a] * (float)(1 << g);
+#pragma unroll
+				for (int q = 0; q < 3; ++q) x[(3 * a + q) >> 2][(3 * a + q) & 3] = tri(p * (float)(1 << (4 * q)));
+			} else {
+				float s[6], c[6];
+				sincos_octaves<6>(rec[a], s, c);
+				x[(3 * a) >> 2][(3 * a) & 3] = pick(s[0], s[1], s[2], s[3]);
+				x[(3 * a + 1) >> 2][(3 * a + 1) & 3] = pick(s[4], s[5], c[0], c[1]);
+				x[(3 * a + 2) >> 2][(3 * a + 2) & 3] = pick(c[2], c[3], c[4], c[5]);
+			}
 		}
-		o[c] = acc;
+		const float k0 = 0.25f * (float)g, k1 = k0 + 0.25f; // the knots of bin g
+#pragma unroll
+		for (int b = 0; b < 5; ++b) {
+			const float u = b == 4 ? 1.0f - expf(-rec[7]) : rec[3 + b];
+			x[(9 + b) >> 2][(9 + b) & 3] = quartic_cdf(k1 - u) - quartic_cdf(k0 - u);
+		}
+		x[3][2] = pick(rec[8], rec[9], rec[10], rec[11]);
+		x[3][3] = pick(rec[12], rec[13], 1.0f, 1.0f);
 	}
 }
 
-// All weights into LDS by a BLOCK-thread block; loads go out four at a time
-// before their LDS stores (one memory round trip per four float4 per thread).
-template <int H, int BLOCK> __device__ __forceinline__ void stage_weights(float *sW, const float *__restrict__ w32) {
-	constexpr int kVec = weight_count(H) / 4;
-	const float4 *src = reinterpret_cast<const float4 *>(w32);
-	float4 *dst = reinterpret_cast<float4 *>(sW);
+// y = relu(W_l x) of this wave's 16 records (NN_nv.glsl:99-127); four independent
+// accumulator chains, one 16-byte LDS read per four MFMAs
+template <int H> __device__ __forceinline__ void layer_forward(const PlainSmem<H> &S, int l, int slot, const float4_t *x, float4_t *y) {
+	float4_t acc[4];
 #pragma unroll
-	for (int b = 0; b < kVec; b += 4 * BLOCK) {
-		const int j0 = b + threadIdx.x, j1 = j0 + BLOCK, j2 = j0 + 2 * BLOCK, j3 = j0 + 3 * BLOCK;
-		float4 v0 = {}, v1 = {}, v2 = {}, v3 = {};
-		if (j0 < kVec) v0 = src[j0];
-		if (j1 < kVec) v1 = src[j1];
-		if (j2 < kVec) v2 = src[j2];
-		if (j3 < kVec) v3 = src[j3];
-		if (j0 < kVec) dst[j0] = v0;
-		if (j1 < kVec) dst[j1] = v1;
-		if (j2 < kVec) dst[j2] = v2;
-		if (j3 < kVec) dst[j3] = v3;
+	for (int m = 0; m < 4; ++m) acc[m] = (float4_t)0.0f;
+#pragma unroll
+	for (int mt = 0; mt < 4; ++mt) {
+		float4_t a[4];
+#pragma unroll
+		for (int m = 0; m < 4; ++m) a[m] = S.frag[((l * 4 + m) * 4 + mt) * 64 + slot];
+#pragma unroll
+		for (int i = 0; i < 4; ++i)
+#pragma unroll
+			for (int m = 0; m < 4; ++m) acc[m] = mfma4(a[m][i], x[mt][i], acc[m]);
 	}
-	__syncthreads();
+#pragma unroll
+	for (int m = 0; m < 4; ++m) y[m] = relu4(acc[m]);
+}
+
+// o = W_H x (NN_nv.glsl:129-158), padded to 16 rows: lane group 0 holds the outputs
+template <int H> __device__ __forceinline__ float4_t output_forward(const PlainSmem<H> &S, int lane, const float4_t *x) {
+	float4_t acc = (float4_t)0.0f;
+#pragma unroll
+	for (int mt = 0; mt < 4; ++mt) {
+		const float4_t a = S.frag_out[mt * 64 + lane];
+#pragma unroll
+		for (int i = 0; i < 4; ++i) acc = mfma4(a[i], x[mt][i], acc);
+	}
+	return acc;
 }
 
 __device__ __forceinline__ void load_query(const float *__restrict__ q, float *rec) {
@@ -87,138 +162,159 @@ __device__ __forceinline__ void load_query(const float *__restrict__ q, float *r
 	}
 }
 
-// nrc_inference.comp:30-48 (without the scene unpack and the epilogue).
+// nrc_inference.comp:30-48 (without the scene unpack and the epilogue).  Persistent, one
+// workgroup a CU, 16-record tiles dealt to the waves in turn.  Bound by the FP32 MFMA
+// rate: 336 MFMAs of 32 cycles a tile, 4.5 us of a SIMD.  230,400
+// queries: 203 -> 85 us (41 -> 112 TFLOP/s) against one thread a query on the vector unit.
 template <int H, int ENC>
-__global__ __launch_bounds__(512) void plain_infer_kernel(const float *__restrict__ queries,
-                                                          const uint32_t *__restrict__ d_count, uint32_t max_count,
-                                                          const float *__restrict__ w32, float *__restrict__ rgb) {
-	__shared__ __attribute__((aligned(16))) float sW[weight_count(H)];
-	stage_weights<H, 512>(sW, w32);
+__global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const float *__restrict__ queries,
+                                                                       const uint32_t *__restrict__ d_count,
+                                                                       uint32_t max_count,
+                                                                       const float *__restrict__ w32,
+                                                                       float *__restrict__ rgb) {
+	__shared__ PlainSmem<H> S;
+	stage_weights<H>(S, w32);
 	const uint32_t count = effective_count(d_count, max_count, max_count);
-	const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-	if (n >= count) return;
-	float rec[kQueryFloats];
-	load_query(queries + (size_t)n * kQueryFloats, rec);
-	float x[kWidth], o[kOut];
-	encode_all<ENC>(rec, x);
-	forward_f32<H>(sW, x, o);
+	const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, slot = 16 * g + ((r + g) & 15);
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint32_t tiles = (count + 15) / 16;
+	for (uint32_t t = wave * gridDim.x + blockIdx.x; t < tiles; t += kPlainWaves * gridDim.x) {
+		const uint32_t n = t * 16 + r, last = count - 1;
+		float rec[kQueryFloats];
+		load_query(queries + (size_t)(n < last ? n : last) * kQueryFloats, rec);
+		float4_t x[4];
+		encode_lane<ENC>(rec, g, x);
+#pragma unroll 1
+		for (int l = 0; l < H; ++l) layer_forward<H>(S, l, slot, x, x);
+		const float4_t o = output_forward<H>(S, lane, x);
+		if (g == 0 && n < count)
 #pragma unroll
-	for (int c = 0; c < kOut; ++c) rgb[(size_t)n * kOut + c] = fmaxf(o[c], 0.0f); // nrc_inference.comp:48
+			for (int c = 0; c < kOut; ++c) rgb[(size_t)n * kOut + c] = fmaxf(o[c], 0.0f); // nrc_inference.comp:48
+	}
 }
 
 // Per record: encode, forward keeping a_0..a_H, loss gradient, then the
 // backward recurrence delta_{l-1} = (W_l^T delta_l) . 1[a_l > 0]
-// (nrc_gradient.comp:26-58, NN_nv.glsl:162-278).  Writes the activations and
-// deltas feature-major so the chunk reduction reads them coalesced.
+// (nrc_gradient.comp:26-58, NN_nv.glsl:162-278).  Writes the activations and deltas of a
+// tile as one 4 KB block [64 features][16 records] a layer, so that every store here and
+// every load of the reduction is a contiguous 256 or 1024 bytes a wave (rows of a whole
+// batch put each load on 16 lines 64 KB apart: the reduction took 25.7 us instead of 17.7).
+// The records that pad the last tile are written as zeros, and the records of a tile are
+// stored in the order 4 (r & 3) + (r >> 2) that the reduction reads.  Bound by the FP32 MFMA rate
+// (592 of 32 cycles a tile for H = 5, 7.9 us of a SIMD; 16,384 records are one tile a
+// SIMD) and the 46 MB of activations and deltas written.
+// 16,384 records: 397 -> 25.7 us against one thread a record (64 workgroups on 256 CUs,
+// a broadcast LDS read a product).
 template <int H, int ENC, int LOSS>
-__global__ __launch_bounds__(256) void plain_fwdbwd_kernel(const float *__restrict__ records,
+__global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const float *__restrict__ records,
                                                            const uint32_t *__restrict__ d_count, uint32_t max_count,
                                                            uint32_t clamp, const float *__restrict__ w32,
                                                            const DeviceState *__restrict__ st, int parity,
                                                            float *__restrict__ acts, float *__restrict__ deltas,
                                                            float *__restrict__ sample_loss, uint32_t ldn) {
-	__shared__ __attribute__((aligned(16))) float sW[weight_count(H)];
-	stage_weights<H, 256>(sW, w32);
+	__shared__ PlainSmem<H> S;
+	stage_weights<H>(S, w32);
 	const uint32_t count = effective_count(d_count, max_count, clamp);
-	const uint32_t n = blockIdx.x * blockDim.x + threadIdx.x;
-	if (n >= count) return;
+	const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, slot = 16 * g + ((r + g) & 15);
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint32_t tiles = (count + 15) / 16;
 	const size_t slab = (size_t)kWidth * ldn;
 	const float s = st->pub[parity].loss_scale;
-	const float *r = records + (size_t)n * kTrainFloats;
-	float rec[kQueryFloats];
+	// floats of W_l^T: row 16 mt + 4 i + g, column 16 Mt + 4 (r & 3) + (r >> 2) of W_l lies
+	// in block (mt, Mt) at slot tslot(i), component r & 3
+	const int gp = r >> 2;
+	int tslot[4];
 #pragma unroll
-	for (int i = 0; i < kQueryFloats; ++i) rec[i] = r[i];
-	const float tgt[3] = {r[14], r[15], r[16]};
-
-	float x[kWidth];
-	encode_all<ENC>(rec, x);
+	for (int i = 0; i < 4; ++i) tslot[i] = (16 * gp + ((4 * g + i + gp) & 15)) * 4 + (r & 3);
+	const float *sf = reinterpret_cast<const float *>(S.frag);
+	for (uint32_t t = wave * gridDim.x + blockIdx.x; t < tiles; t += kPlainWaves * gridDim.x) {
+		const uint32_t n = t * 16 + r, last = count - 1;
+		const bool valid = n < count;
+		const float *rp = records + (size_t)(valid ? n : last) * kTrainFloats;
+		float rec[kTrainFloats];
 #pragma unroll
-	for (int k = 0; k < kWidth; ++k) acts[k * ldn + n] = x[k];
-#pragma unroll 1
-	for (int l = 0; l < H; ++l) {
-		const float *Wl = sW + l * kWidth * kWidth;
-		float y[kWidth];
+		for (int i = 0; i < kTrainFloats; ++i) rec[i] = rp[i];
+		// features 16 mt + 4 i + g of this lane's record in the tile's block of a slab
+		const size_t blk = (size_t)t * (16 * kWidth) + 4 * (r & 3) + (r >> 2);
+		auto store = [&](float *dst, const float4_t *v) __attribute__((always_inline)) {
 #pragma unroll
-		for (int m = 0; m < kWidth; ++m) {
-			float acc = 0.0f;
+			for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-			for (int k = 0; k < kWidth; k += 4) {
-				const float4 w = *reinterpret_cast<const float4 *>(Wl + m * kWidth + k);
-				acc = fmaf(w.x, x[k + 0], acc);
-				acc = fmaf(w.y, x[k + 1], acc);
-				acc = fmaf(w.z, x[k + 2], acc);
-				acc = fmaf(w.w, x[k + 3], acc);
-			}
-			y[m] = fmaxf(acc, 0.0f);
+				for (int i = 0; i < 4; ++i) dst[blk + 16 * (16 * mt + 4 * i + g)] = v[mt][i];
+		};
+		float4_t a[H + 1][4];
+		encode_lane<ENC>(rec, g, a[0]);
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+			for (int i = 0; i < 4; ++i) a[0][mt][i] = valid ? a[0][mt][i] : 0.0f;
+		store(acts, a[0]);
+#pragma unroll
+		for (int l = 0; l < H; ++l) {
+			layer_forward<H>(S, l, slot, a[l], a[l + 1]);
+			store(acts + (size_t)(l + 1) * slab, a[l + 1]);
 		}
-		float *al = acts + (size_t)(l + 1) * slab;
+		const float4_t ov = output_forward<H>(S, lane, a[H]);
+		const float o[kOut] = {__shfl(ov[0], r), __shfl(ov[1], r), __shfl(ov[2], r)}; // from lane group 0
+		float go[kOut];
+		const float v = loss_grad<LOSS>(o, rec + kQueryFloats, s, go);
 #pragma unroll
-		for (int m = 0; m < kWidth; ++m) {
-			x[m] = y[m];
-			al[m * ldn + n] = y[m];
+		for (int c = 0; c < kOut; ++c) go[c] = valid ? go[c] : 0.0f;
+		if (g == 0) {
+			sample_loss[n] = valid ? v : 0.0f;
+			float *dH = deltas + (size_t)H * slab;
+#pragma unroll
+			for (int c = 0; c < kOut; ++c) dH[blk + 16 * c] = go[c];
 		}
-	}
-	const float *Wo = sW + H * kWidth * kWidth;
-	float o[kOut];
-#pragma unroll
-	for (int c = 0; c < kOut; ++c) {
-		float acc = 0.0f;
-#pragma unroll
-		for (int k = 0; k < kWidth; ++k) acc = fmaf(Wo[c * kWidth + k], x[k], acc);
-		o[c] = acc;
-	}
-	float go[kOut];
-	sample_loss[n] = loss_grad<LOSS>(o, tgt, s, go);
-	float *dH = deltas + (size_t)H * slab;
-#pragma unroll
-	for (int c = 0; c < kOut; ++c) dH[c * ldn + n] = go[c];
 
-	// delta_{H-1} = (W_H^T g_o) . 1[a_H > 0]   (NNBackwardDA3_ReLU, NN_nv.glsl:222-246)
-	float g[kWidth];
+		// delta_{H-1} = (W_H^T g_o) . 1[a_H > 0]   (NNBackwardDA3_ReLU, NN_nv.glsl:222-246)
+		float4_t d[4];
 #pragma unroll
-	for (int k = 0; k < kWidth; ++k) {
-		float v = Wo[k] * go[0];
-		v = fmaf(Wo[kWidth + k], go[1], v);
-		v = fmaf(Wo[2 * kWidth + k], go[2], v);
-		g[k] = relu_bwd(v, x[k]);
-	}
-	{
-		float *d = deltas + (size_t)(H - 1) * slab;
+		for (int mt = 0; mt < 4; ++mt) {
+			const float4_t *w = S.frag_out + mt * 64 + 16 * g; // W_H[c][16 mt + 4 i + g] at lane row c
+			const float4_t w0 = w[0], w1 = w[1], w2 = w[2];
 #pragma unroll
-		for (int k = 0; k < kWidth; ++k) d[k * ldn + n] = g[k];
-	}
-	// delta_{l-1} = (W_l^T delta_l) . 1[a_l > 0], l = H-1..1  (NNBackwardDA64_ReLU, NN_nv.glsl:248-278)
-#pragma unroll 1
-	for (int l = H - 1; l >= 1; --l) {
-		const float *Wl = sW + l * kWidth * kWidth;
-		float gn[kWidth];
-#pragma unroll
-		for (int k = 0; k < kWidth; ++k) gn[k] = 0.0f;
-#pragma unroll
-		for (int m = 0; m < kWidth; ++m) {
-#pragma unroll
-			for (int k = 0; k < kWidth; k += 4) {
-				const float4 w = *reinterpret_cast<const float4 *>(Wl + m * kWidth + k);
-				gn[k + 0] = fmaf(w.x, g[m], gn[k + 0]);
-				gn[k + 1] = fmaf(w.y, g[m], gn[k + 1]);
-				gn[k + 2] = fmaf(w.z, g[m], gn[k + 2]);
-				gn[k + 3] = fmaf(w.w, g[m], gn[k + 3]);
+			for (int i = 0; i < 4; ++i) {
+				float y = w0[i] * go[0];
+				y = fmaf(w1[i], go[1], y);
+				y = fmaf(w2[i], go[2], y);
+				d[mt][i] = relu_bwd(y, a[H][mt][i]);
 			}
 		}
-		const float *al = acts + (size_t)l * slab;
-		float *d = deltas + (size_t)(l - 1) * slab;
+		store(deltas + (size_t)(H - 1) * slab, d);
+		// delta_{l-1} = (W_l^T delta_l) . 1[a_l > 0], l = H-1..1  (NNBackwardDA64_ReLU, NN_nv.glsl:248-278)
 #pragma unroll
-		for (int k = 0; k < kWidth; ++k) {
-			g[k] = relu_bwd(gn[k], al[k * ldn + n]);
-			d[k * ldn + n] = g[k];
+		for (int l = H - 1; l >= 1; --l) {
+			float4_t acc[4];
+#pragma unroll
+			for (int m = 0; m < 4; ++m) acc[m] = (float4_t)0.0f;
+#pragma unroll
+			for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+				for (int i = 0; i < 4; ++i)
+#pragma unroll
+					for (int m = 0; m < 4; ++m)
+						acc[m] = mfma4(sf[((l * 4 + mt) * 4 + m) * 256 + tslot[i]], d[mt][i], acc[m]);
+#pragma unroll
+			for (int m = 0; m < 4; ++m)
+#pragma unroll
+				for (int i = 0; i < 4; ++i) d[m][i] = relu_bwd(acc[m][i], a[l][m][i]);
+			store(deltas + (size_t)(l - 1) * slab, d);
 		}
 	}
 }
 
 // Partial dW over one chunk of records: dW_l[m][k] = sum_n delta_l[m][n] a_l[k][n]
-// (NNUpdateDW64 / NNUpdateDW3, NN_nv.glsl:280-367).  Grid: x over blocks of 256
-// weights (one layer, four output rows each), y over chunks.  Also writes the
-// chunk's loss sum after the weights and flags non-finite partials.
+// (NNUpdateDW64 / NNUpdateDW3, NN_nv.glsl:280-367), the records in order.  Grid: x over
+// half layers (32 output units) and the output layer, y over chunks; a wave computes two of
+// the 16x16 tiles as dW^T (A = activations, B = deltas, K = records, so a lane stores four
+// consecutive inputs), reading 16 bytes of a feature a lane straight from memory: in
+// the stored order a lane group's float4 holds records 4 j + g, the K index g of step j.
+// The loads of the next 64 records are in flight while the MFMAs of 64 run.  Also writes
+// the chunk's loss sum after the weights and flags non-finite partials.  Bound by the
+// reads of what the kernel before wrote (46 MB for 16,384 records, past the L2s) more than
+// by its MFMAs (256 a wave, 3.4 us).  16,384 records: 65 -> 17.7 us against
+// FMAs from LDS tiles.
 template <int H>
 __global__ __launch_bounds__(256) void plain_dw_kernel(const uint32_t *__restrict__ d_count, uint32_t max_count,
                                                        uint32_t clamp, const float *__restrict__ acts,
@@ -227,47 +323,71 @@ __global__ __launch_bounds__(256) void plain_dw_kernel(const uint32_t *__restric
                                                        float *__restrict__ partials, uint32_t pstride,
                                                        uint32_t *__restrict__ overflow) {
 	constexpr int WC = weight_count(H);
-	__shared__ float sa[kWidth][kWidth + 1];
-	__shared__ float sd[4][kWidth];
-	__shared__ float sl[256];
 	const uint32_t count = effective_count(d_count, max_count, clamp);
-	const int t = threadIdx.x;
-	const uint32_t w0 = blockIdx.x * 256u;
-	const int l = (int)(w0 / (kWidth * kWidth));
-	const int m0 = (int)((w0 % (kWidth * kWidth)) / kWidth);
-	const int rows = (l == H) ? kOut : 4;
-	const int mr = t / kWidth, k = t % kWidth;
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int g = lane >> 4, r = lane & 15;
+	const bool output = blockIdx.x == 2 * H;
+	const int l = (int)blockIdx.x >> 1; // H for the output layer
 	const size_t slab = (size_t)kWidth * ldn;
-	const float *a = acts + (size_t)l * slab;
-	const float *d = deltas + (size_t)l * slab;
 	const uint32_t nb0 = blockIdx.y * kPlainChunk;
 	uint32_t nend = nb0 + kPlainChunk;
 	if (nend > count) nend = count;
-	float acc = 0.0f;
-	for (uint32_t nb = nb0; nb < nend; nb += kWidth) {
-		// stage a_l[0..63][nb..nb+63] and delta_l[m0..m0+3][nb..nb+63]
-#pragma unroll
-		for (int i = 0; i < 16; ++i) {
-			const int e = t + 256 * i;
-			const int kk = e / kWidth, j = e % kWidth;
-			sa[kk][j] = (nb + j < nend) ? a[kk * ldn + nb + j] : 0.0f;
-		}
-		{
-			const int rr = t / kWidth, j = t % kWidth;
-			sd[rr][j] = (rr < rows && nb + j < nend) ? d[(m0 + rr) * ldn + nb + j] : 0.0f;
-		}
-		__syncthreads();
-#pragma unroll 8
-		for (int j = 0; j < kWidth; ++j) acc = fmaf(sd[mr][j], sa[k][j], acc);
-		__syncthreads();
-	}
-	const uint32_t w = w0 + (uint32_t)t;
 	float *pp = partials + (size_t)blockIdx.y * pstride;
-	if (w < (uint32_t)WC) {
-		pp[w] = acc;
-		if (!isfinite(acc)) atomicOr(overflow, 1u);
-	}
-	if (blockIdx.x == 0) {
+	bool bad = false;
+	auto put = [&](float *dst, float4_t v) __attribute__((always_inline)) {
+		*reinterpret_cast<float4_t *>(dst) = v;
+#pragma unroll
+		for (int i = 0; i < 4; ++i) bad |= !isfinite(v[i]);
+	};
+	// NA input tiles from it0 against output tile ot (or, LAST, the three output rows)
+	auto tiles = [&](auto na, auto last, int it0, int ot) __attribute__((always_inline)) {
+		constexpr int NA = decltype(na)::value, STEPS = 4; // 16-record steps in flight
+		constexpr bool LAST = decltype(last)::value;
+		const bool live = !LAST || r < kOut;
+		const float *a = acts + (size_t)l * slab + 16 * (16 * it0 + r) + 4 * g;
+		const float *d = deltas + (size_t)l * slab + 16 * (16 * ot + (live ? r : 0)) + 4 * g;
+		float4_t acc[NA];
+#pragma unroll
+		for (int i = 0; i < NA; ++i) acc[i] = (float4_t)0.0f;
+		if (nb0 < nend) {
+			const uint32_t lastn = (nend - 1) & ~15u; // the last 16-record step
+			float4_t av[2][STEPS][NA], dv[2][STEPS];
+			auto load = [&](int b, uint32_t nb) __attribute__((always_inline)) {
+#pragma unroll
+				for (int k = 0; k < STEPS; ++k) {
+					const uint32_t n = nb + 16 * k < lastn ? nb + 16 * k : lastn;
+#pragma unroll
+					for (int i = 0; i < NA; ++i) av[b][k][i] = *reinterpret_cast<const float4_t *>(a + (size_t)n * kWidth + 256 * i);
+					dv[b][k] = *reinterpret_cast<const float4_t *>(d + (size_t)n * kWidth);
+				}
+			};
+			auto run = [&](int b, uint32_t nb) __attribute__((always_inline)) {
+#pragma unroll
+				for (int k = 0; k < STEPS; ++k)
+					if (nb + 16 * k < nend) // uniform
+#pragma unroll
+						for (int j = 0; j < 4; ++j)
+#pragma unroll
+							for (int i = 0; i < NA; ++i) acc[i] = mfma4(av[b][k][i][j], live ? dv[b][k][j] : 0.0f, acc[i]);
+			};
+			load(0, nb0);
+			for (uint32_t nb = nb0; nb < nend; nb += 32 * STEPS) {
+				load(1, nb + 16 * STEPS);
+				run(0, nb);
+				load(0, nb + 32 * STEPS);
+				run(1, nb + 16 * STEPS);
+			}
+		}
+		if (live)
+#pragma unroll
+			for (int i = 0; i < NA; ++i) put(pp + l * kWidth * kWidth + (16 * ot + r) * kWidth + 16 * (it0 + i) + 4 * g, acc[i]);
+	};
+	if (!output) {
+		tiles(std::integral_constant<int, 2>{}, std::false_type{}, 2 * (wave & 1), 2 * ((int)blockIdx.x & 1) + (wave >> 1));
+	} else {
+		tiles(std::integral_constant<int, 1>{}, std::true_type{}, wave, 0);
+		__shared__ float sl[256];
+		const int t = threadIdx.x;
 		float v = 0.0f;
 		for (uint32_t n = nb0 + t; n < nend; n += 256) v += sample_loss[n];
 		sl[t] = v;
@@ -278,6 +398,7 @@ __global__ __launch_bounds__(256) void plain_dw_kernel(const uint32_t *__restric
 		}
 		if (t == 0) pp[WC] = sl[0];
 	}
+	if (__any(bad) && lane == 0) atomicOr(overflow, 1u);
 }
 
 template <int ENC>
@@ -303,10 +424,16 @@ __global__ __launch_bounds__(256) void sph_kernel(const float *__restrict__ dirs
 	uv[2 * i + 1] = o[1];
 }
 
+// One workgroup a CU, and no more than there are tiles.
+uint32_t plain_blocks(uint32_t n) {
+	const uint32_t tiles = (n + 15) / 16, cus = (uint32_t)device_cu_count();
+	return tiles < cus ? tiles : cus;
+}
+
 template <int H>
 hipError_t plain_infer_h(int enc, const float *q, const uint32_t *dc, uint32_t mc, const float *w, float *rgb,
                          hipStream_t s) {
-	const dim3 grid((mc + 511) / 512), block(512);
+	const dim3 grid(plain_blocks(mc)), block(64 * kPlainWaves);
 	switch (enc) {
 	case NRC_ENCODING_TRI12: plain_infer_kernel<H, NRC_ENCODING_TRI12><<<grid, block, 0, s>>>(q, dc, mc, w, rgb); break;
 	case NRC_ENCODING_SINCOS6: plain_infer_kernel<H, NRC_ENCODING_SINCOS6><<<grid, block, 0, s>>>(q, dc, mc, w, rgb); break;
@@ -316,7 +443,7 @@ hipError_t plain_infer_h(int enc, const float *q, const uint32_t *dc, uint32_t m
 }
 
 template <int H, int ENC, int LOSS> void plain_fwdbwd_launch(const TrainArgs &a, hipStream_t s) {
-	const dim3 grid((a.max_count + 255) / 256), block(256);
+	const dim3 grid(plain_blocks(a.max_count < a.clamp ? a.max_count : a.clamp)), block(64 * kPlainWaves);
 	plain_fwdbwd_kernel<H, ENC, LOSS><<<grid, block, 0, s>>>(a.records, a.d_count, a.max_count, a.clamp, a.w32,
 	                                                          a.state, a.parity, a.acts, a.deltas, a.sample_loss, a.ldn);
 }
@@ -332,7 +459,7 @@ template <int H> void plain_gradient_h(const TrainArgs &a, uint32_t nparts, hipS
 	case NRC_ENCODING_SINCOS6: plain_fwdbwd_loss<H, NRC_ENCODING_SINCOS6>(a, s); break;
 	default: plain_fwdbwd_loss<H, NRC_ENCODING_UV_SINCOS16>(a, s); break;
 	}
-	const dim3 grid((weight_count(H) + 255) / 256, nparts), block(256);
+	const dim3 grid(2 * H + 1, nparts), block(256);
 	plain_dw_kernel<H><<<grid, block, 0, s>>>(a.d_count, a.max_count, a.clamp, a.acts, a.deltas, a.sample_loss, a.ldn,
 	                                          a.partials, a.pstride, &a.state->overflow[a.parity]);
 }
