@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import vknrc_amd as v
+from oracle.fp8 import infer_fp8
 from oracle.oracle import Oracle
 from vknrc_amd import workloads as wl
 
@@ -133,3 +134,35 @@ def test_plain_gradient_chunks(hidden, enc, n, live):
     assert rel_err(s["m"] / (1.0 - np.float32(0.9)), G / live) < PLAIN_GRAD_TOL
     assert abs(s["state"]["last_loss"] / (loss / live) - 1) < PLAIN_GRAD_TOL
     st.close()
+
+
+# the FP8 tiles: one to a few records of a 32-record half, both halves, one tile and one more, and
+# a workgroup's worth of tiles; every size gives the records the bits they have in a large call
+# (whose parity with the FP8 oracle is tests/test_gpu_fp8.py's), and nothing past the count is written
+@pytest.mark.parametrize("hidden,enc", ENCODINGS)
+def test_fp8_inference_tiles(hidden, enc):
+    w, r = plain_inputs(hidden, enc, 4097)
+    r[:, 3:8] = np.linspace(-0.5, 1.5, r[:, 3:8].size, dtype=np.float32).reshape(-1, 5)  # every one-blob knot
+
+    def first(n, live):
+        st = v.NRCState(v.NRCConfig(hidden_layers=hidden, encoding=enc))
+        st.set_state(weight=w)
+        out = torch.full((n, 3), 7.0, device=DEV)
+        st.infer(dev(r[:n, :14]), out, count=dev(np.array([live], np.uint32).view(np.int32)), path=v.PATH_FUSED_F8)
+        y = host(out)
+        st.close()
+        return y
+
+    whole = first(4097, 4097)
+    f = Oracle("f32").encode(r, enc)
+    st = v.NRCState(v.NRCConfig(hidden_layers=hidden, encoding=enc))
+    st.set_state(weight=w)
+    st.infer(dev(r[:, :14]), torch.zeros((4097, 3), device=DEV), path=v.PATH_FUSED_F8)
+    sc = st.get_fp8_scales()
+    st.close()
+    # 5e-2: an e4m3 step is 6-12 % of a value, and sums near a rounding boundary fall either way
+    assert rel_err(whole, infer_fp8(f, w, hidden, sc["layer_scales"], sc["out_scale"], clamp0=True)) < 5e-2
+    for n, live in ((1, 1), (31, 31), (33, 33), (64, 63), (65, 65), (257, 257), (1025, 900)):
+        y = first(n, live)
+        assert np.array_equal(y[:live], whole[:live]), n
+        assert (y[live:] == 7.0).all()

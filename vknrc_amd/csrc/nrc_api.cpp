@@ -145,7 +145,7 @@ nrc_status reset_cache(nrc_cache *c, uint64_t seed) {
 	NRC_HIP(nrc::launch_init_state(c->state, c->desc.loss_scale, nullptr), "init state");
 	// FP8: no scales and no activation history yet; the padding of the fp8 copy stays zero
 	NRC_HIP(hipMemset(c->f8, 0, sizeof(nrc::Fp8State)), "init fp8 state");
-	NRC_HIP(hipMemset(c->w8, 0, (size_t)nrc::fwd_frag_halves((int)c->desc.hidden_layers)), "init fp8 weights");
+	NRC_HIP(hipMemset(c->w8, 0, (size_t)nrc::fp8_frag_bytes((int)c->desc.hidden_layers)), "init fp8 weights");
 	c->parity = 0;
 	NRC_HIP(hipDeviceSynchronize(), "reset");
 	c->desc.seed = seed;
@@ -432,7 +432,7 @@ struct CacheSizes {
 		w16 = use16 = 2 * wc;
 		wf = usef = 2 * (size_t)nrc::fwd_frag_halves(H);
 		wtf = 2 * (size_t)nrc::bwd_frag_halves(H);
-		w8 = (size_t)nrc::fwd_frag_halves(H);
+		w8 = (size_t)nrc::fp8_frag_bytes(H);
 		f8 = sizeof(nrc::Fp8State);
 		w32 = use32 = 4 * wc;
 		state = sizeof(DeviceState);

@@ -40,6 +40,18 @@ template <typename T> __host__ __device__ inline void frag_scatter(uint32_t i, T
 	if (wtf && l >= 1) wtf[frag_pos(l - 1, col, row)] = h;
 }
 
+// Fragment-major e4m3 use-weights, the A operands of the FP8 inference's
+// v_mfma_f32_32x32x16_fp8_fp8: block b = 8 * layer + 4 * m + c holds 64 lanes x 8 bytes,
+// lane 32h + r carrying row 32m + r at the columns
+//   32 (c >> 1) + 8 (c & 1) + 4h + (j & 3) + 16 (j >> 2)
+// and the output layer in blocks 8H .. 8H+3 (rows 3..31 stay zero).
+__host__ __device__ constexpr uint32_t fp8_frag_bytes(int hidden) { return (uint32_t)(hidden * 8 + 4) * 512u; }
+// Position of element (row, col) of layer l; columns 4k .. 4k+3 are consecutive bytes.
+__host__ __device__ inline uint32_t fp8_frag_pos(uint32_t l, uint32_t row, uint32_t col) {
+	const uint32_t block = (l * 2u + (row >> 5)) * 4u + ((col >> 5) << 1) + ((col >> 3) & 1u);
+	return (block * 64u + ((col >> 2) & 1u) * 32u + (row & 31u)) * 8u + (col & 3u) + ((col >> 4) & 1u) * 4u;
+}
+
 // Device-resident optimizer state, double-buffered by a parity the host flips
 // on every launched train step: step p reads pub[p] and writes pub[p ^ 1], and
 // its gradient kernels flag non-finite partials in overflow[p] (the optimizer

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 				}
 			} else {
 				if (n < count) {
-					encode_quads<ENC, true>(rec, emit);
+					encode_quads<ENC>(rec, emit);
 				} else {
 #pragma unroll
 					for (int p = 0; p < 16; ++p) emit(p, 0.0f, 0.0f, 0.0f, 0.0f);
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 		float ra[kQueryFloats], rb[kQueryFloats];
 		load_query(lt0, ra);
 		load_query(lt0 + 1, rb);
-		encode_quads<ENC, true>(ra, emitter(slot0));
+		encode_quads<ENC>(ra, emitter(slot0));
 		wave_lds_sync();
 		for (uint32_t t = lt0; t < lt1; t += 2) {
 			load_query(t + 2, ra);

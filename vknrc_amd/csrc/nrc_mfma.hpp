@@ -84,9 +84,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 //   * one-blob (NRCOneBlob4Encode, NRCRecord.glsl:51-63): per knot k = 0..4,
 //     c_k = clamp(0.5 + u (15/16 - 5/8 u^2 + 3/16 u^4), 0, 1) with u = k - 4x,
 //     which is (15/16) u (1 - (2/3) u^2 + (1/5) u^4) + 0.5 in Horner form
-//     (6 instructions a knot instead of 11; oneblob4_knots, which the FP8 kernel
-//     uses); the FP16 kernels evaluate only the two unsaturated knots and place
-//     the packed quad with byte permutes (oneblob4_packed);
+//     (6 instructions a knot instead of 11); only the two unsaturated knots are evaluated,
+//     and the packed quad is placed with byte permutes (oneblob4_packed, oneblob4_fp8);
 //   * SINCOS6: sin/cos(2^k pi p) for k = 0..5 from one polynomial evaluation at
 //     k = 0 and five double-angle steps (largest error 1.3e-5 at k = 5, a twentieth
 //     of an FP16 half-ulp at 1);
@@ -94,22 +93,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 //     2 |mod(a, 2) - 1| - 1 is |4 fract(a/2) - 2| - 1, the same value (every step
 //     scales by a power of two or rounds once in both) except where fract clamps
 //     a result that rounds to 1 down to 1 - 2^-24.
-__device__ __forceinline__ void oneblob4_knots(float x, float *o) {
-	const float x4 = 4.0f * x;
-	float c[5];
-#pragma unroll
-	for (int k = 0; k < 5; ++k) {
-		const float u = (float)k - x4;
-		const float u2 = u * u;
-		float t = fmaf(u2, 0.1875f, -0.625f);
-		t = fmaf(u2, t, 0.9375f);
-		c[k] = fminf(fmaxf(fmaf(u, t, 0.5f), 0.0f), 1.0f);
-	}
-#pragma unroll
-	for (int b = 0; b < 4; ++b) o[b] = c[b + 1] - c[b];
-}
-
-// The same one-blob quad with two knots, packed to FP16.  With j = floor(4x) and
+// The one-blob quad from two knots, packed to FP16.  With j = floor(4x) and
 // f = 4x - j (exact), only knots j and j+1 have |u| < 1: c_j = C(-f), c_{j+1} =
 // C(1 - f), every knot below j is 0 and every one above j+1 is 1.  So the quad holds
 // c_j, c_{j+1} - c_j and 1 - c_{j+1} at positions j-1, j and j+1 and zeros elsewhere.
@@ -165,6 +149,36 @@ __device__ __forceinline__ uint2 oneblob4_packed(float x, const uint2 *sel) {
 	return make_uint2(__builtin_amdgcn_perm(hi, lo, s.x), __builtin_amdgcn_perm(hi, lo, s.y));
 }
 
+// four values -> four e4m3 bytes (first value in the low byte)
+__device__ __forceinline__ uint32_t pack4_fp8(float a, float b, float c, float d) {
+	// the first conversion keeps the upper half of its old value, which the second replaces:
+	// a's own register serves (a zero would have to be moved in first)
+	int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, __float_as_int(a), false);
+	w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
+	return (uint32_t)w;
+}
+
+// The same quad as e4m3 bytes: one byte permute of (c_j, c_{j+1} - c_j, 1 - c_{j+1}, 0)
+// with the selectors of kOneBlobSel8.  The knots it leaves out change a feature by 6e-8 at
+// most (above), which is 0 in e4m3 (smallest value 2^-9).
+constexpr uint32_t kOneBlobSel8[8] = {0x0C0C0C0Cu, 0x0C0C0C02u, 0x0C0C0201u, 0x0C020100u,
+                                      0x0201000Cu, 0x01000C0Cu, 0x000C0C0Cu, 0x0C0C0C0Cu};
+
+__device__ __forceinline__ void oneblob_sel8_init(uint32_t *tab, int lane) {
+	if (lane < 8) tab[lane] = kOneBlobSel8[lane];
+}
+
+__device__ __forceinline__ uint32_t oneblob4_fp8(float x, const uint32_t *sel) {
+	const float x4 = 4.0f * x;
+	const float j = __builtin_floorf(x4);
+	const float f = x4 - j;
+	const float c0 = quartic_cdf(-f), c1 = quartic_cdf(1.0f - f);
+	const uint32_t q = pack4_fp8(c0, c1 - c0, 1.0f - c1, 0.0f);
+	int k = (int)j; // saturating, NaN -> 0, as in oneblob4_packed
+	k = k < -2 ? -2 : (k > 5 ? 5 : k);
+	return __builtin_amdgcn_perm(0u, q, sel[k + 2]);
+}
+
 template <int ENC> __device__ __forceinline__ void axis12_infer(float p, float *o) {
 	if constexpr (ENC == NRC_ENCODING_SINCOS6) {
 		float sv, cv;
@@ -187,10 +201,9 @@ template <int ENC> __device__ __forceinline__ void axis12_infer(float p, float *
 		}
 	}
 }
-// Emits the 16 feature quads (features 4p..4p+3) of one record; Emit(p, f0..f3).
-// PACKED: the one-blob quads come from oneblob4_packed through Emit.bits(p, halves)
-// with the selector table Emit.sel (the FP16 kernels); otherwise from the five knots.
-template <int ENC, bool PACKED = false, typename Emit> __device__ __forceinline__ void encode_quads(const float *rec, Emit &&emit) {
+// Emits the 16 feature quads (features 4p..4p+3) of one record: Emit(p, f0..f3), and
+// Emit.oneblob(p, x) for the one-blob quads.
+template <int ENC, typename Emit> __device__ __forceinline__ void encode_quads(const float *rec, Emit &&emit) {
 	if constexpr (ENC == NRC_ENCODING_UV_SINCOS16) {
 #pragma unroll
 		for (int a = 0; a < 2; ++a) {
@@ -222,24 +235,15 @@ template <int ENC, bool PACKED = false, typename Emit> __device__ __forceinline_
 			emit(3 * a + 1, t[4], t[5], t[6], t[7]);
 			emit(3 * a + 2, t[8], t[9], t[10], t[11]);
 		}
-		if constexpr (PACKED) {
 #pragma unroll
-			for (int q = 0; q < 5; ++q) emit.bits(9 + q, oneblob4_packed(q == 4 ? 1.0f - expf(-rec[7]) : rec[3 + q], emit.sel));
-		} else {
-			float b[4];
-#pragma unroll
-			for (int q = 0; q < 5; ++q) {
-				oneblob4_knots(q == 4 ? 1.0f - expf(-rec[7]) : rec[3 + q], b);
-				emit(9 + q, b[0], b[1], b[2], b[3]);
-			}
-		}
+		for (int q = 0; q < 5; ++q) emit.oneblob(9 + q, q == 4 ? 1.0f - expf(-rec[7]) : rec[3 + q]);
 		emit(14, rec[8], rec[9], rec[10], rec[11]);
 		emit(15, rec[12], rec[13], 1.0f, 1.0f);
 	}
 }
 
 
-// The same quads in pieces (the one-blob quads packed, as encode_quads<ENC, true>), so
+// The same quads in pieces, so
 // that the encoding of one tile can be spread over the layers of another: piece P of
 // encode_pieces<ENC>() emits
 //   TRI12 / SINCOS6:  P = 0..2 the 12 features of position axis P (quads 3P..3P+2),
@@ -272,7 +276,7 @@ template <int ENC, int P, typename Emit> __device__ __forceinline__ void encode_
 		emit(3 * P + 1, t[4], t[5], t[6], t[7]);
 		emit(3 * P + 2, t[8], t[9], t[10], t[11]);
 	} else if constexpr (P < 8) {
-		emit.bits(6 + P, oneblob4_packed(P == 7 ? 1.0f - expf(-rec[7]) : rec[P], emit.sel));
+		emit.oneblob(6 + P, P == 7 ? 1.0f - expf(-rec[7]) : rec[P]);
 	} else {
 		emit(14, rec[8], rec[9], rec[10], rec[11]);
 		emit(15, rec[12], rec[13], 1.0f, 1.0f);
@@ -292,7 +296,7 @@ struct SlotEmit {
 		h[0] = (_Float16)f0; h[1] = (_Float16)f1; h[2] = (_Float16)f2; h[3] = (_Float16)f3;
 		s4[at(p)] = h;
 	}
-	__device__ __forceinline__ void bits(int p, uint2 v) const { s4[at(p)] = __builtin_bit_cast(half4_t, v); }
+	__device__ __forceinline__ void oneblob(int p, float x) const { s4[at(p)] = __builtin_bit_cast(half4_t, oneblob4_packed(x, sel)); }
 };
 
 // feature index of element j of a B operand held by lane group g for K-chunk c
