@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import vknrc_amd as v
+from oracle import frontend
 from oracle.fp8 import infer_fp8
 from oracle.oracle import Oracle
 from vknrc_amd import workloads as wl
@@ -166,3 +167,39 @@ def test_fp8_inference_tiles(hidden, enc):
         y = first(n, live)
         assert np.array_equal(y[:live], whole[:live]), n
         assert (y[live:] == 7.0).all()
+
+
+# the unpack takes 64 records a wave through LDS, four lanes fetching one record's scene data:
+# every lane of a partial wave, one wave and one record more, a device count inside a wave, odd
+# record addresses; each prefix gives the rows of the whole, and nothing past the count is written
+@pytest.mark.parametrize("packed", [False, True])
+def test_unpack_partial_waves(packed):
+    s = wl.make_scene(5, primitives=300, vertices=200, instances=3, materials=5, textures=2, texture_size=16)
+    ds = v.DeviceScene(torch, s["vertices"], s["vertex_indices"], s["texcoords"], s["texcoord_indices"], s["materials"],
+                       s["material_ids"], s["transforms"], s["textures"])
+    if packed:
+        ds.pack_primitives()
+    rng = np.random.default_rng(6)
+    ev = np.zeros(700, v.EVAL_RECORD)
+    ev["packed_input"] = wl.make_packed_inputs(s, 700, rng)
+    tr = np.zeros(700, v.WIRE_TRAIN_RECORD)
+    tr["packed_input"], tr["bias"] = ev["packed_input"], rng.uniform(0, 1, (700, 3))
+    ref = frontend.unpack(s, ev["packed_input"])
+    words = lambda a: dev(np.concatenate([np.zeros(1, np.int32), np.frombuffer(a.tobytes(), np.int32)]))[1:]  # noqa: E731
+
+    def rows(fn, rec, width, n, live):
+        out = torch.full((n, width), 7.0, device=DEV)
+        fn(ds, words(rec[:n]), n, out, count=dev(np.array([live], np.uint32).view(np.int32)))
+        y = host(out)
+        assert (y[live:] == 7.0).all()
+        return y[:live]
+
+    whole = rows(v.unpack_eval_records, ev, 14, 700, 700)
+    # 2e-5 is FP32 rounding of positions and colours of order 1; the sphere encoding's acos is steep at its poles
+    assert np.abs(whole - ref)[:, [0, 1, 2, 3, 4, 7, 8, 9, 10, 11, 12, 13]].max() < 2e-5
+    assert np.quantile(np.abs(whole - ref)[:, 5:7], 0.99) < 1e-5
+    trained = rows(v.unpack_train_records, tr, 17, 700, 700)
+    assert np.array_equal(trained[:, :14], whole) and np.array_equal(trained[:, 14:], tr["bias"])
+    for n, live in ((1, 1), (3, 2), (63, 63), (64, 64), (65, 65), (256, 255), (257, 257), (600, 321)):
+        assert np.array_equal(rows(v.unpack_eval_records, ev, 14, n, live), whole[:live]), n
+        assert np.array_equal(rows(v.unpack_train_records, tr, 17, n, live), trained[:live]), n

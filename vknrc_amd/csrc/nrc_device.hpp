@@ -75,6 +75,16 @@ __device__ __forceinline__ uint32_t effective_count(const uint32_t *d_count, uin
 	return c < clamp ? c : clamp;
 }
 
+// Orders LDS traffic between lanes of one wavefront (LDS operations of a wave
+// execute in order; this keeps the compiler from moving them across).  The
+// fences are restricted to LDS so they wait on LDS counters only and leave the
+// prefetched global loads in flight.
+__device__ __forceinline__ void wave_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // ---------------------------------------------------------------- encoders
 // _nrc_tri, NRCRecord.glsl:65-68 with GLSL's floor-based mod(a, 2).
 __device__ __forceinline__ float tri(float x) {
@@ -250,11 +260,19 @@ __device__ __forceinline__ float mul_add_rn(float b, float f, float p) {
 	return b + m;
 }
 
+// x / c for a constant c: the product with the rounded reciprocal and one remainder step,
+// 3 instructions where the general division takes about 10 (its scaling covers quotients
+// out of range, which c and x of ordinary size do not have).
+__device__ __forceinline__ float div_const(float x, float c) {
+	const float q = x * (1.0f / c);
+	return fmaf(fmaf(-q, c, x), 1.0f / c, q);
+}
+
 // NRCSphEncode, NRCRecord.glsl:47-49.
 __device__ __forceinline__ void sph_encode(float x, float y, float z, float *uv) {
 	constexpr float kPi = 3.14159265358979323846f;
-	uv[0] = (x == 0.0f && y == 0.0f) ? 0.5f : 0.5f + atan2f(y, x) / (2.0f * kPi);
-	uv[1] = acosf(fminf(fmaxf(z, -1.0f), 1.0f)) / kPi;
+	uv[0] = (x == 0.0f && y == 0.0f) ? 0.5f : 0.5f + div_const(atan2f(y, x), 2.0f * kPi);
+	uv[1] = div_const(acosf(fminf(fmaxf(z, -1.0f), 1.0f)), kPi);
 }
 
 // ReLU backward with the reference's NaN-mask semantics (NN_nv.glsl:198-220,

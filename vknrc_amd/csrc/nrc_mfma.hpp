@@ -67,16 +67,6 @@ template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
 	static_for_seq(f, std::make_integer_sequence<int, N>{});
 }
 
-// Orders LDS traffic between lanes of one wavefront (LDS operations of a wave
-// execute in order; this keeps the compiler from moving them across).  The
-// fences are restricted to LDS so they wait on LDS counters only and leave the
-// prefetched global loads in flight.
-__device__ __forceinline__ void wave_lds_sync() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-
 // --------------------------------------------------------------- encoders
 // The inference kernels round the features to FP16 (or e4m3) right away, so they
 // use shorter forms of two encoders than the FP32 restatements in nrc_device.hpp,

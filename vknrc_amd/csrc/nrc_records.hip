@@ -6,6 +6,8 @@
 //
 // All four are gathers and streams over HBM with a few dozen FLOPs a record, one
 // thread per record (or pixel); the MLP kernels read the unpacked 56-byte queries.
+#include <cstddef>
+
 #include "nrc_internal.hpp"
 
 namespace nrc {
@@ -14,10 +16,11 @@ namespace {
 
 constexpr uint32_t kNoTexture = 0xFFFFFFFFu;
 
-// unpackUnorm2x16: c / 65535 per 16-bit half
+// unpackUnorm2x16: c / 65535 per 16-bit half (div_const gives the correctly rounded
+// quotient for every one of the 65,536 values)
 __device__ __forceinline__ void unorm2x16(uint32_t v, float *o) {
-	o[0] = (float)(v & 0xFFFFu) / 65535.0f;
-	o[1] = (float)(v >> 16) / 65535.0f;
+	o[0] = div_const((float)(v & 0xFFFFu), 65535.0f);
+	o[1] = div_const((float)(v >> 16), 65535.0f);
 }
 
 __device__ __forceinline__ float srgb_decode(uint32_t c8) {
@@ -80,37 +83,69 @@ __device__ __forceinline__ void material_color(const nrc_scene &s, const float *
 	}
 }
 
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef f4v __attribute__((aligned(4))) f4v_any;
+
+// The 16-byte pieces 0 .. PIECES-1 of record `index` of this lane, from 64 lanes' records of
+// `stride` bytes at any 4-byte alignment.  Four neighbouring lanes fetch one record, so a
+// load instruction touches 16 lines instead of 64 (the vector cache looks up a line or so a
+// cycle, which bounds these gathers), and the pieces go to their lanes through the wave's
+// 4 KB of LDS, pieces rotated by lane so that neither side conflicts on banks.  Every lane
+// of the wave takes part; a lane without a record passes some valid index.
+template <int PIECES>
+__device__ __forceinline__ void gather_records(const void *base, uint32_t stride, uint32_t index, int lane, f4v *buf, f4v *out) {
+	const int piece = lane & 3;
+	f4v v[4];
+#pragma unroll
+	for (int k = 0; k < 4; ++k) {
+		const uint32_t i = (uint32_t)__shfl((int)index, 16 * k + (lane >> 2));
+		if (piece < PIECES)
+			v[k] = *reinterpret_cast<const f4v_any *>(static_cast<const char *>(base) + (size_t)i * stride + 16 * piece);
+	}
+#pragma unroll
+	for (int k = 0; k < 4; ++k) {
+		const int rec = 16 * k + (lane >> 2);
+		if (piece < PIECES) buf[rec * 4 + (piece ^ ((rec >> 2) & 3))] = v[k];
+	}
+	wave_lds_sync();
+#pragma unroll
+	for (int j = 0; j < PIECES; ++j) out[j] = buf[lane * 4 + (j ^ ((lane >> 2) & 3))];
+	wave_lds_sync();
+}
+
 // A primitive's corners (object space), their texture coordinates and its material:
 // gathered through the index arrays (Scene.glsl:50-62), or read from the primitive's
-// 64-byte packed record (nrc_scene_pack_primitives) as four 16-byte loads.
+// 64-byte packed record (nrc_scene_pack_primitives).
 struct PrimitiveData {
 	float c[3][3], t[3][2];
 	uint32_t material;
 };
 
-template <bool PACKED> __device__ __forceinline__ PrimitiveData load_primitive(const nrc_scene &s, uint32_t prim) {
+__device__ __forceinline__ PrimitiveData indexed_primitive(const nrc_scene &s, uint32_t prim) {
 	PrimitiveData d;
-	if constexpr (PACKED) {
-		const float4 *r = reinterpret_cast<const float4 *>(s.d_primitives + prim);
-		const float4 a = r[0], b = r[1], c = r[2], e = r[3];
-		d.c[0][0] = a.x; d.c[0][1] = a.y; d.c[0][2] = a.z;
-		d.c[1][0] = a.w; d.c[1][1] = b.x; d.c[1][2] = b.y;
-		d.c[2][0] = b.z; d.c[2][1] = b.w; d.c[2][2] = c.x;
-		d.t[0][0] = c.y; d.t[0][1] = c.z;
-		d.t[1][0] = c.w; d.t[1][1] = e.x;
-		d.t[2][0] = e.y; d.t[2][1] = e.z;
-		d.material = __float_as_uint(e.w);
-	} else {
 #pragma unroll
-		for (int k = 0; k < 3; ++k) {
-			const uint32_t vi = s.d_vertex_indices[prim * 3u + k], ti = s.d_texcoord_indices[prim * 3u + k];
+	for (int k = 0; k < 3; ++k) {
+		const uint32_t vi = s.d_vertex_indices[prim * 3u + k], ti = s.d_texcoord_indices[prim * 3u + k];
 #pragma unroll
-			for (int j = 0; j < 3; ++j) d.c[k][j] = s.d_vertices[(size_t)vi * 3 + j];
-			d.t[k][0] = s.d_texcoords[(size_t)ti * 2];
-			d.t[k][1] = s.d_texcoords[(size_t)ti * 2 + 1];
-		}
-		d.material = s.d_material_ids[prim];
+		for (int j = 0; j < 3; ++j) d.c[k][j] = s.d_vertices[(size_t)vi * 3 + j];
+		d.t[k][0] = s.d_texcoords[(size_t)ti * 2];
+		d.t[k][1] = s.d_texcoords[(size_t)ti * 2 + 1];
 	}
+	d.material = s.d_material_ids[prim];
+	return d;
+}
+
+__device__ __forceinline__ PrimitiveData packed_primitive(const f4v *r) {
+	PrimitiveData d;
+	const f4v a = r[0], b = r[1], c = r[2], e = r[3];
+	d.c[0][0] = a[0]; d.c[0][1] = a[1]; d.c[0][2] = a[2];
+	d.c[1][0] = a[3]; d.c[1][1] = b[0]; d.c[1][2] = b[1];
+	d.c[2][0] = b[2]; d.c[2][1] = b[3]; d.c[2][2] = c[0];
+	d.t[0][0] = c[1]; d.t[0][1] = c[2];
+	d.t[1][0] = c[3]; d.t[1][1] = e[0];
+	d.t[2][0] = e[1]; d.t[2][1] = e[2];
+	const float m = e[3];
+	d.material = __float_as_uint(m);
 	return d;
 }
 
@@ -120,13 +155,32 @@ __device__ __forceinline__ void transform_vertex(const float *T, const float *v,
 	for (int j = 0; j < 3; ++j) o[j] = T[4 * j] * v[0] + T[4 * j + 1] * v[1] + T[4 * j + 2] * v[2] + T[4 * j + 3];
 }
 
-// UnpackNRCInput (NRCRecord.glsl:98-125) into the 14 floats of an nrc_query
+// UnpackNRCInput (NRCRecord.glsl:98-125) into the 14 floats of an nrc_query; `buf` is the
+// wave's 4 KB of LDS, and every lane of the wave calls this
 template <bool PACKED>
-__device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, const float *lut, float *q) {
+__device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, const float *lut, int lane, f4v *buf, float *q) {
 	const uint32_t prim = p.primitive_id, inst = p.flip_bit_instance_id & 0x7FFFFFFFu;
 	const bool flip = (p.flip_bit_instance_id >> 31) != 0u;
-	const PrimitiveData d = load_primitive<PACKED>(s, prim);
-	const float *T = s.d_transforms + (size_t)inst * 12;
+	PrimitiveData d;
+	if constexpr (PACKED) {
+		f4v r[4];
+		gather_records<4>(s.d_primitives, 64u, prim, lane, buf, r);
+		d = packed_primitive(r);
+	} else {
+		d = indexed_primitive(s, prim);
+	}
+	// opaque values, so that the compiler fuses the products below into the sums in the same
+	// way whichever way they were loaded: the packed records give the bits of the index arrays
+#pragma unroll
+	for (int k = 0; k < 3; ++k) {
+		asm volatile("" : "+v"(d.c[k][0]), "+v"(d.c[k][1]), "+v"(d.c[k][2]));
+		asm volatile("" : "+v"(d.t[k][0]), "+v"(d.t[k][1]));
+	}
+	f4v rows[3], mat[4];
+	gather_records<3>(s.d_transforms, 48u, inst, lane, buf, rows);
+	gather_records<4>(s.d_materials, 64u, d.material, lane, buf, mat);
+	const float T[12] = {rows[0][0], rows[0][1], rows[0][2], rows[0][3], rows[1][0], rows[1][1],
+	                     rows[1][2], rows[1][3], rows[2][0], rows[2][1], rows[2][2], rows[2][3]};
 	float v0[3], v1[3], v2[3];
 	transform_vertex(T, d.c[0], v0);
 	transform_vertex(T, d.c[1], v1);
@@ -146,13 +200,18 @@ __device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, cons
 	for (int j = 0; j < 3; ++j) q[j] = v0[j] * b[0] + v1[j] * b[1] + v2[j] * b[2];
 	unorm2x16(p.scattered_dir_2x16u, q + 3);
 	sph_encode(n[0], n[1], n[2], q + 5);
-	const nrc_material &m = s.d_materials[d.material];
-	q[7] = m.roughness;
+	const float diffuse[3] = {mat[0][0], mat[0][1], mat[0][2]}, specular[3] = {mat[1][0], mat[1][1], mat[1][2]};
+	const float dt = mat[0][3], st = mat[1][3];
+	q[7] = mat[3][1]; // roughness
 	const float u = d.t[0][0] * b[0] + d.t[1][0] * b[1] + d.t[2][0] * b[2];
 	const float v = d.t[0][1] * b[0] + d.t[1][1] * b[1] + d.t[2][1] * b[2];
-	material_color(s, m.diffuse, m.diffuse_texture_id, u, v, lut, q + 8);
-	material_color(s, m.specular, m.specular_texture_id, u, v, lut, q + 11);
+	material_color(s, diffuse, __float_as_uint(dt), u, v, lut, q + 8);
+	material_color(s, specular, __float_as_uint(st), u, v, lut, q + 11);
 }
+static_assert(offsetof(nrc_material, diffuse_texture_id) == 12 && offsetof(nrc_material, specular) == 16 &&
+                  offsetof(nrc_material, specular_texture_id) == 28 && offsetof(nrc_material, roughness) == 52 &&
+                  sizeof(nrc_material) == 64,
+              "the material fields that unpack_input picks from 16-byte pieces");
 
 __device__ __forceinline__ nrc_packed_input load_packed(const uint32_t *w) {
 	nrc_packed_input p;
@@ -163,51 +222,59 @@ __device__ __forceinline__ nrc_packed_input load_packed(const uint32_t *w) {
 	return p;
 }
 
-template <bool PACKED>
-__global__ __launch_bounds__(256) void unpack_eval_kernel(const nrc_scene s, const nrc_eval_record *__restrict__ rec,
-                                                          const uint32_t *d_count, uint32_t max_count,
-                                                          float *__restrict__ out) {
+// Unpacks wire records of WORDS dwords, whose packed input starts at dword AT, into rows of
+// FLOATS floats (queries, or training records with the record's bias as the target,
+// nrc_gradient.comp:30-33).  A wave's 64 records come in and its rows go out through its LDS
+// as contiguous dwords (any 4-byte alignment), where a record a lane straight from and to
+// memory touched 10 to 56 lines an instruction.  Bound by the vector cache's line look-ups
+// (8 a record, 14.5 without the shared gathers), the vector unit (690 instructions a
+// record) and the misses of L2 (1.3 a record), each busy for about 60 % of the time.
+// 2,073,600 eval records on random packed primitives: 80.3 -> 67 us.
+constexpr uint32_t kUnpackWaves = 4;
+template <bool PACKED, int WORDS, int AT, int FLOATS>
+__global__ __launch_bounds__(64 * kUnpackWaves) void unpack_kernel(const nrc_scene s, const uint32_t *__restrict__ rec,
+                                                     const uint32_t *d_count, uint32_t max_count,
+                                                     float *__restrict__ out) {
 	__shared__ float lut[256];
+	constexpr int kWaveWords = 64 * (FLOATS > 16 ? FLOATS : 16); // records in, then gathers, then rows out
+	__shared__ __attribute__((aligned(16))) uint32_t stage[kUnpackWaves][kWaveWords];
+	static_assert(WORDS <= 16, "the records fit the stage");
 	srgb_table_init(lut);
-	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-	if (i >= effective_count(d_count, max_count, max_count)) return;
-	const uint32_t *w = reinterpret_cast<const uint32_t *>(rec + i);
-	float q[kQueryFloats];
-	unpack_input<PACKED>(s, load_packed(w + 1), lut, q);
-	float2 *o = reinterpret_cast<float2 *>(out + (size_t)i * kQueryFloats);
+	const uint32_t count = effective_count(d_count, max_count, max_count);
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	uint32_t *const st = stage[wave];
+	const uint32_t first = (blockIdx.x * kUnpackWaves + (uint32_t)wave) * 64u;
+	if (first >= count) return; // uniform over the wave
+	const uint32_t n = count - first < 64u ? count - first : 64u;
+	const uint32_t *src = rec + (size_t)first * WORDS;
 #pragma unroll
-	for (int k = 0; k < kQueryFloats / 2; ++k) o[k] = make_float2(q[2 * k], q[2 * k + 1]);
-}
-
-template <bool PACKED>
-__global__ __launch_bounds__(256) void unpack_train_kernel(const nrc_scene s,
-                                                           const nrc_wire_train_record *__restrict__ rec,
-                                                           const uint32_t *d_count, uint32_t max_count,
-                                                           float *__restrict__ out) {
-	__shared__ float lut[256];
-	srgb_table_init(lut);
-	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-	if (i >= effective_count(d_count, max_count, max_count)) return;
-	const uint32_t *w = reinterpret_cast<const uint32_t *>(rec + i);
-	float q[kTrainFloats];
-	unpack_input<PACKED>(s, load_packed(w + 6), lut, q);
-	// nrc_gradient.comp:30-33: the target is the record's bias
-	q[14] = __uint_as_float(w[0]);
-	q[15] = __uint_as_float(w[1]);
-	q[16] = __uint_as_float(w[2]);
-	float *o = out + (size_t)i * kTrainFloats;
+	for (int k = 0; k < WORDS; ++k)
+		if (lane + 64u * k < n * WORDS) st[lane + 64u * k] = src[lane + 64u * k];
+	wave_lds_sync();
+	const uint32_t *w = st + ((uint32_t)lane < n ? (uint32_t)lane : n - 1u) * WORDS; // a lane past the count repeats the last record
+	const nrc_packed_input p = load_packed(w + AT);
+	float q[FLOATS];
 #pragma unroll
-	for (int k = 0; k < kTrainFloats; ++k) o[k] = q[k];
+	for (int k = kQueryFloats; k < FLOATS; ++k) q[k] = __uint_as_float(w[k - kQueryFloats]);
+	wave_lds_sync();
+	unpack_input<PACKED>(s, p, lut, lane, reinterpret_cast<f4v *>(st), q);
+#pragma unroll
+	for (int k = 0; k < FLOATS; ++k) st[lane * FLOATS + k] = __float_as_uint(q[k]);
+	wave_lds_sync();
+	uint32_t *dst = reinterpret_cast<uint32_t *>(out) + (size_t)first * FLOATS;
+#pragma unroll
+	for (int k = 0; k < FLOATS; ++k)
+		if (lane + 64u * k < n * FLOATS) dst[lane + 64u * k] = st[lane + 64u * k];
 }
 
 // One thread per primitive: the corners and texture coordinates its indices name and
-// its material id, in the 64-byte record that load_primitive<true> reads (16-float
+// its material id, in the 64-byte record that packed_primitive reads (16-float
 // order: corners 0..2 xyz, texcoords 0..2 uv, material id bits).
 __global__ __launch_bounds__(256) void pack_primitives_kernel(const nrc_scene s, uint32_t n,
                                                               nrc_scene_primitive *__restrict__ out) {
 	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
 	if (i >= n) return;
-	const PrimitiveData d = load_primitive<false>(s, i);
+	const PrimitiveData d = indexed_primitive(s, i);
 	float4 *o = reinterpret_cast<float4 *>(out + i);
 	o[0] = make_float4(d.c[0][0], d.c[0][1], d.c[0][2], d.c[1][0]);
 	o[1] = make_float4(d.c[1][1], d.c[1][2], d.c[2][0], d.c[2][1]);
@@ -356,24 +423,30 @@ hipError_t launch_pack_primitives(const nrc_scene &s, uint32_t n, nrc_scene_prim
 	return hipGetLastError();
 }
 
+namespace {
+template <int WORDS, int AT, int FLOATS>
+hipError_t launch_unpack(const nrc_scene &s, const void *rec, const uint32_t *d_count, uint32_t max_count, float *out,
+                         hipStream_t stream) {
+	if (max_count == 0) return hipSuccess;
+	const dim3 grid((max_count + 64u * kUnpackWaves - 1u) / (64u * kUnpackWaves)), block(64 * kUnpackWaves);
+	const uint32_t *r = static_cast<const uint32_t *>(rec);
+	if (s.d_primitives)
+		unpack_kernel<true, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out);
+	else
+		unpack_kernel<false, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out);
+	return hipGetLastError();
+}
+static_assert(sizeof(nrc_eval_record) == 20 && sizeof(nrc_wire_train_record) == 40, "wire records in dwords");
+} // namespace
+
 hipError_t launch_unpack_eval(const nrc_scene &s, const nrc_eval_record *rec, const uint32_t *d_count,
                               uint32_t max_count, float *queries, hipStream_t stream) {
-	if (max_count == 0) return hipSuccess;
-	if (s.d_primitives)
-		unpack_eval_kernel<true><<<dim3((max_count + 255) / 256), dim3(256), 0, stream>>>(s, rec, d_count, max_count, queries);
-	else
-		unpack_eval_kernel<false><<<dim3((max_count + 255) / 256), dim3(256), 0, stream>>>(s, rec, d_count, max_count, queries);
-	return hipGetLastError();
+	return launch_unpack<5, 1, kQueryFloats>(s, rec, d_count, max_count, queries, stream);
 }
 
 hipError_t launch_unpack_train(const nrc_scene &s, const nrc_wire_train_record *rec, const uint32_t *d_count,
                                uint32_t max_count, float *out, hipStream_t stream) {
-	if (max_count == 0) return hipSuccess;
-	if (s.d_primitives)
-		unpack_train_kernel<true><<<dim3((max_count + 255) / 256), dim3(256), 0, stream>>>(s, rec, d_count, max_count, out);
-	else
-		unpack_train_kernel<false><<<dim3((max_count + 255) / 256), dim3(256), 0, stream>>>(s, rec, d_count, max_count, out);
-	return hipGetLastError();
+	return launch_unpack<10, 6, kTrainFloats>(s, rec, d_count, max_count, out, stream);
 }
 
 hipError_t launch_composite_records(const float *rgb, const nrc_eval_record *rec, const uint32_t *d_count,
