@@ -203,3 +203,39 @@ def test_unpack_partial_waves(packed):
     for n, live in ((1, 1), (3, 2), (63, 63), (64, 64), (65, 65), (256, 255), (257, 257), (600, 321)):
         assert np.array_equal(rows(v.unpack_eval_records, ev, 14, n, live), whole[:live]), n
         assert np.array_equal(rows(v.unpack_train_records, tr, 17, n, live), trained[:live]), n
+
+
+# more multi-chunk rows than CUs run two a workgroup: caches with an odd number of rows, a single
+# row, a partial last chunk, device counts that leave a row's last chunk or whole rows empty, and a
+# chunk whose deltas carry a scale, each with the bits that the cache has alone
+@pytest.mark.parametrize("hidden,enc", ENCODINGS)
+@pytest.mark.parametrize("loss", [v.LOSS_RELATIVE_L2_LUMINANCE, v.LOSS_L2])
+def test_gradient_row_pairs(hidden, enc, loss):
+    sizes = [(16384, 16384, 2), (16383, 16383, 2), (12000, 7001, 3), (64, 64, 2), (16384, 100, 2), (16000, 0, 4),
+             (8257, 8257, 2)]
+    assert sum(-(-n // (64 * c)) for n, _, c in sizes) > 256
+
+    def caches():
+        out = []
+        for i, (n, live, chunks) in enumerate(sizes):
+            w, r = plain_inputs(hidden, enc, n)
+            if i == 1:
+                r[200:230, 14:] *= 1e6
+            st = v.NRCState(v.NRCConfig(hidden_layers=hidden, encoding=enc, loss=loss))
+            st.set_state(weight=w)
+            st.set_grad_chunks(chunks)
+            out.append(dict(cache=st, batches=dev(r), max_batch_records=n,
+                            batch_counts=dev(np.array([live], np.uint32).view(np.int32))))
+        return out
+
+    group, alone = caches(), caches()
+    v.group_train(group, 0, write_use_weights=True)
+    for e in alone:
+        e["cache"].train(e["batches"], count=e["batch_counts"], max_count=e["max_batch_records"])
+    for g, a in zip(group, alone):
+        x, y = g["cache"].get_state(), a["cache"].get_state()
+        for k in ("weight", "m", "v", "ema_weight", "weights_f16", "use_weights_f16"):
+            assert np.array_equal(x[k], y[k]), k
+        assert x["state"] == y["state"]
+    for e in group + alone:
+        e["cache"].close()

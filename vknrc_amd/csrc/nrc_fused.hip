@@ -902,6 +902,356 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 	if (overflow && __any(bad) && lane == 0) atomicOr(overflow, 1u);
 }
 
+// The gradient for launches with more multi-chunk rows than CUs: a workgroup of 8 waves, two a
+// SIMD, computes two rows of one cache side by side (waves 0-3 the first, 4-7 the second),
+// each as fused_grad_small_kernel computes it and with its sums in the same order, so a row
+// has the same bits from either kernel.  With one wave a SIMD nothing hides the latency of a
+// row's chain (its matrix cores are 14 % busy, its vector unit 40 %); two rows a CU hide
+// each other's.  To fit two rows in a CU, LDS holds the activations of both, one delta buffer
+// a row and one copy of the weights that serves both rows and both directions, 158 KB.  dW is
+// taken layer by layer in the backward, the deltas alternating between the buffer and the rows
+// of a_H, free once the output layer's dW is taken.  The weights lie as forward A fragments,
+// each split in its two 4-half runs (256 halves of a block, then 256): the forward reads both
+// runs, 512 contiguous bytes each, and the backward's W_l^T fragments come from transposing
+// reads of one run, which also touch 512 contiguous bytes.  (Forward fragments read from L1
+// and L2 one layer ahead instead, 42 KB a wave and chunk, took 72 us where this takes 67.)
+// Bound by LDS: about 1.1 MB a chunk of both rows (fragments, activations, dW operands), then
+// the chain's latency.  293 rows of 8 chunks (16 caches): 85.2 -> 67 us.
+template <int H> struct DualGradSmem {
+	_Float16 w[(H * 8 + 2) * 512]; // forward A fragments: [block][run][16 g + r][4]
+	struct Row {
+		_Float16 act[H + 1][kFusedSmallRecords * kRowLd]; // a_l; [H]: later delta_{H-1}, delta_{H-3}
+		_Float16 dlt[kFusedSmallRecords * kRowLd];        // delta_H, delta_{H-2}, ..
+		_Float16 go[kFusedSmallRecords * kGoLd];          // output gradient
+		float lsum[4];
+		float gmax[4]; // largest |output gradient| of each wave's records
+	} row[2];
+};
+
+template <int H, int ENC, int LOSS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void fused_grad_dual_kernel(
+    const GradGroup grp) {
+	// this workgroup's cache, as in fused_grad_small_kernel
+	uint32_t k = 0;
+#pragma unroll
+	for (uint32_t j = 1; j < (uint32_t)kGroupMax; ++j)
+		k += (j < grp.n_items && blockIdx.x >= grp.item[j].block_begin) ? 1u : 0u;
+	const GradItem &gi = grp.item[k];
+	const uint32_t blk0 = 2 * (blockIdx.x - gi.block_begin); // the workgroup's first row
+	const float *__restrict__ records = gi.records;
+	const uint32_t nch = gi.chunks, pstride = gi.pstride;
+	const DeviceState *__restrict__ st = gi.state;
+	constexpr int WC = weight_count(H);
+	constexpr int R = (int)kFusedSmallRecords;
+	extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+	DualGradSmem<H> &D = *reinterpret_cast<DualGradSmem<H> *>(smem_raw);
+
+	// wave-uniform values are kept in SGPRs; `wave` is the wave's index within its row
+	const int tid = threadIdx.x, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3;
+	auto &S = D.row[wave8 >> 2];
+	int lane = tid & 63;
+	int g = lane >> 4, r = lane & 15;
+	int col = 16 * wave + r; // record column this lane runs through the network
+	const uint32_t blk = blk0 + (uint32_t)(wave8 >> 2);
+	const uint32_t count = effective_count(gi.d_count, gi.max_count, gi.clamp);
+	const uint32_t span = nch * (uint32_t)R, base0 = blk * span, first0 = blk0 * span;
+	float *part = gi.partials + (size_t)blk * pstride;
+	const int it0 = 2 * (wave & 1), ot0 = 2 * (wave >> 1); // this wave's dW tiles
+
+	bool bad = false;
+	auto store_tile = [&](int l, int it, int ot, float4_t v) __attribute__((always_inline)) {
+		__builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(part + l * kWidth * kWidth + (16 * ot + r) * kWidth + 16 * it + 4 * g));
+#pragma unroll
+		for (int e = 0; e < 4; ++e) bad |= !isfinite(v[e]);
+	};
+	auto store_out_tile = [&](float4_t v) __attribute__((always_inline)) {
+		if (r < kOut) {
+			__builtin_nontemporal_store(v, reinterpret_cast<float4_t *>(part + H * kWidth * kWidth + r * kWidth + 16 * wave + 4 * g));
+#pragma unroll
+			for (int e = 0; e < 4; ++e) bad |= !isfinite(v[e]);
+		}
+	};
+	float4_t accW[H][2][2], accO = (float4_t)0.0f; // dW tiles summed over the chunks
+#pragma unroll
+	for (int l = 0; l < H; ++l)
+#pragma unroll
+		for (int i = 0; i < 2; ++i) accW[l][i][0] = accW[l][i][1] = (float4_t)0.0f;
+	// this wave's tiles of its row (the second row of an odd count does not exist)
+	auto store_row = [&]() __attribute__((always_inline)) {
+		if (blk >= gi.blocks) return;
+#pragma unroll
+		for (int l = 0; l < H; ++l)
+#pragma unroll
+			for (int i = 0; i < 2; ++i)
+#pragma unroll
+				for (int o = 0; o < 2; ++o) store_tile(l, it0 + i, ot0 + o, accW[l][i][o]);
+		store_out_tile(accO);
+	};
+	if (first0 >= count) { // uniform: no valid record in this workgroup, so its partial rows are zero
+		store_row();
+		if (wave == 0 && lane == 0 && blk < gi.blocks) part[WC] = 0.0f;
+		return;
+	}
+	// records at or past the end are invalid: past the count, or past this row's chunks (a
+	// row without a valid record runs as zeros beside the other)
+	const uint32_t end = count < base0 ? base0 : count - base0 < span ? count : base0 + span;
+	const float scale = st == nullptr ? 1.0f : st->pub[gi.parity].loss_scale;
+	const uint32_t last = (end > base0 ? end : count) - 1;
+
+	float q[kQueryFloats];
+	float tg[3];
+	// the inputs this lane encodes and the targets of the record it runs; the next chunk's
+	// are loaded once this chunk's are used, and are in flight during the rest of the chunk
+	auto load_inputs = [&](uint32_t base) __attribute__((always_inline)) {
+		const uint32_t n_enc = base + lane < last ? base + lane : last;
+		const float *rp = records + (size_t)n_enc * kTrainFloats;
+#pragma unroll
+		for (int i = 0; i < kQueryFloats; ++i) q[i] = rp[i];
+	};
+	auto load_targets = [&](uint32_t base) __attribute__((always_inline)) {
+		const uint32_t n_run = base + col < last ? base + col : last;
+		const float *tp = records + (size_t)n_run * kTrainFloats + kQueryFloats;
+#pragma unroll
+		for (int e = 0; e < 3; ++e) tg[e] = tp[e];
+	};
+	load_inputs(base0);
+	load_targets(base0);
+	// the weights go to LDS once per workgroup, every load in flight before the first store
+	{
+		constexpr int kFrags = (H * 8 + 2) * 64, kPer = (kFrags + 511) / 512;
+		const half8_t *wfv = reinterpret_cast<const half8_t *>(gi.wf);
+		half4_t *w4 = reinterpret_cast<half4_t *>(D.w);
+		half8_t v[kPer];
+#pragma unroll
+		for (int i = 0; i < kPer; ++i) v[i] = wfv[tid + 512 * i < kFrags ? tid + 512 * i : 0];
+#pragma unroll
+		for (int i = 0; i < kPer; ++i) {
+			const int f = tid + 512 * i; // block f >> 6, lane f & 63
+			if (f < kFrags) {
+				w4[(f >> 6) * 128 + (f & 63)] = v[i].lo;
+				w4[(f >> 6) * 128 + 64 + (f & 63)] = v[i].hi;
+			}
+		}
+	}
+	// this lane's forward A fragment of block b
+	auto fwd_frag = [&](int b) __attribute__((always_inline)) {
+		const half4_t *p = reinterpret_cast<const half4_t *>(D.w) + b * 128 + lane;
+		return (half8_t)__builtin_shufflevector(p[0], p[64], 0, 1, 2, 3, 4, 5, 6, 7);
+	};
+	// Columns 16 mt + r of rows 16 m + 4 g + k, k = 0..3, of the layer in slot l.
+	// ds_read_b64_tr_b16 gives lane i of each 16-lane group element i % 4 of the 4 halves that
+	// lane 4 k + i / 4 of the group addresses, as element k; so lane 4 k + q addresses columns
+	// 16 mt + 4 q .. of row 16 m + 4 g + k: run mt & 1 of block 8 l + 2 m + (mt >> 1), lane slot
+	// 16 q + 4 g + k.
+	auto tr_quad = [&](int l, int m, int mt) __attribute__((always_inline)) {
+		typedef short short4_t __attribute__((ext_vector_type(4)));
+		typedef __attribute__((address_space(3))) short4_t lds_short4;
+		const _Float16 *p = D.w + (l * 8 + 2 * m + (mt >> 1)) * 512 + (mt & 1) * 256 + (16 * (r & 3) + 4 * g + (r >> 2)) * 4;
+		return __builtin_bit_cast(half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)p));
+	};
+	// the backward A fragment of W_l^T: M-tile mt, K-chunk c
+	auto bwd_frag = [&](int l, int mt, int c) __attribute__((always_inline)) {
+		return (half8_t)__builtin_shufflevector(tr_quad(l, 2 * c, mt), tr_quad(l, 2 * c + 1, mt), 0, 1, 2, 3, 4, 5, 6, 7);
+	};
+	if (lane == 0) S.lsum[wave] = 0.0f; // the loss sums start at zero
+
+	for (uint32_t ch = 0; ch < nch; ++ch) {
+		const uint32_t base = base0 + ch * (uint32_t)R;
+		if (first0 + ch * (uint32_t)R >= count) break; // uniform over the workgroup: past the first row's records
+		if (ch > 0) block_lds_sync(); // the previous chunk's dW readers are done with the LDS buffers
+		{
+			// recompute the lane-derived indices each chunk from an opaque copy of the
+			// lane id, so the LDS addresses built from them are not kept live across chunks
+			asm volatile("" : "+v"(lane));
+			g = lane >> 4;
+			r = lane & 15;
+			col = 16 * wave + r;
+		}
+		// ---- encode: wave w of a row computes feature block w (features 16w ..) of record base + lane
+		{
+			_Float16 *a0 = S.act[0];
+			const bool valid = base + lane < end;
+			auto put = [&](auto qc) __attribute__((always_inline)) {
+				constexpr int qb = decltype(qc)::value;
+				float f[16];
+				encode_block<ENC>(q, qb, f);
+				half4_t h[4];
+#pragma unroll
+				for (int j = 0; j < 16; ++j) h[j >> 2][j & 3] = valid ? (_Float16)f[j] : (_Float16)0.0f;
+#pragma unroll
+				for (int j = 0; j < 4; ++j) *reinterpret_cast<half4_t *>(a0 + row_at(lane, 16 * qb + 4 * j)) = h[j];
+			};
+			switch (wave) {
+			case 0: put(std::integral_constant<int, 0>{}); break;
+			case 1: put(std::integral_constant<int, 1>{}); break;
+			case 2: put(std::integral_constant<int, 2>{}); break;
+			default: put(std::integral_constant<int, 3>{}); break;
+			}
+		}
+		block_lds_sync();
+		if (ch + 1 < nch) load_inputs(base + R); // the next chunk's inputs (uniform branch)
+
+		// ---- forward for this wave's 16 records
+		half8_t B[2];
+		uint4 keep[H][2]; // ReLU masks of a_1 .. a_{H-1} in B layout, for the backward
+		load_brow(S.act[0], B, g, col);
+		static_for<H>([&](auto l_c) __attribute__((always_inline)) {
+			constexpr int l = decltype(l_c)::value;
+			half8_t A[4][2];
+#pragma unroll
+			for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+				for (int mt = 0; mt < 4; ++mt) A[mt][kc] = fwd_frag((l * 4 + mt) * 2 + kc);
+			float4_t acc[4];
+#pragma unroll
+			for (int mt = 0; mt < 4; ++mt) acc[mt] = (float4_t)0.0f;
+#pragma unroll
+			for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+				for (int mt = 0; mt < 4; ++mt) acc[mt] = mfma(A[mt][kc], B[kc], acc[mt]);
+#pragma unroll
+			for (int kc = 0; kc < 2; ++kc) B[kc] = pack_relu(acc[2 * kc], acc[2 * kc + 1]);
+			if constexpr (l + 1 < H) {
+				keep[l + 1][0] = act_masks(B[0]);
+				keep[l + 1][1] = act_masks(B[1]);
+			}
+			store_brow(S.act[l + 1], B, g, col);
+		});
+		float4_t o = (float4_t)0.0f;
+#pragma unroll
+		for (int kc = 0; kc < 2; ++kc) o = mfma(fwd_frag(H * 8 + kc), B[kc], o);
+
+		// ---- loss gradient: lanes g == 0 hold the 3 outputs of record col
+		float go[3] = {0.0f, 0.0f, 0.0f};
+		float lv = 0.0f, gm = 0.0f;
+		if (g == 0) {
+			const bool valid = base + col < end;
+			const float oo[3] = {o[0], o[1], o[2]};
+			const float v = loss_grad<LOSS>(oo, tg, scale, go);
+			lv = valid ? v : 0.0f;
+#pragma unroll
+			for (int e = 0; e < kOut; ++e) {
+				go[e] = valid ? go[e] : 0.0f;
+				gm = fmaxf(gm, fabsf(go[e]));
+			}
+		}
+		if (ch + 1 < nch) load_targets(base + R); // the next chunk's targets (uniform branch)
+		// The deltas of a chunk share one power-of-two scale 2^k: k = 0 unless its largest
+		// output gradient reaches kDeltaLimit, where FP16 would overflow and force a skipped
+		// step.  Scaling by 2^k is exact.
+#pragma unroll
+		for (int off = 32; off >= 1; off >>= 1) gm = fmaxf(gm, __shfl_xor(gm, off));
+		if (lane == 0) S.gmax[wave] = gm;
+		block_lds_sync();
+		float dscale = 1.0f, undo = 1.0f;
+		{
+			const float wmax = fmaxf(fmaxf(S.gmax[0], S.gmax[1]), fmaxf(S.gmax[2], S.gmax[3]));
+			if (wmax >= kDeltaLimit && wmax <= 3.0e38f) {
+				const int e = 12 - ilogbf(wmax);
+				dscale = ldexpf(1.0f, e);
+				undo = ldexpf(1.0f, -e);
+			}
+		}
+		half8_t Bg = (half8_t)0;
+		if (g == 0) { // the record's whole row: units 0..2, then zeros
+#pragma unroll
+			for (int e = 0; e < kOut; ++e) Bg[e] = (_Float16)(go[e] * dscale);
+			*reinterpret_cast<half8_t *>(S.go + col * kGoLd) = Bg;
+			*reinterpret_cast<half8_t *>(S.go + col * kGoLd + 8) = (half8_t)0;
+		}
+		// dW tiles of this wave, K = a chunk's 64 records (all waves' a_l and delta): the sums
+		// are scaled by the chunk's 2^k before its products and by 2^-k after (exact), behind
+		// a uniform branch, so the scale costs nothing on the chunks that have none
+		auto scaled = [](float4_t *t, int n, float by) __attribute__((always_inline)) {
+			if (by != 1.0f) { // uniform
+				asm volatile("" ::: "memory"); // keeps the multiplies behind the branch
+#pragma unroll
+				for (int i = 0; i < n; ++i) t[i] *= by;
+			}
+		};
+		auto dw_layer = [&](int l, const _Float16 *d) __attribute__((always_inline)) {
+			scaled(&accW[l][0][0], 4, dscale);
+#pragma unroll
+			for (int kc = 0; kc < R / 32; ++kc) {
+				half8_t a[2], b[2];
+#pragma unroll
+				for (int i = 0; i < 2; ++i) {
+					a[i] = load_kop<true, kRowLd>(S.act[l], 16 * (it0 + i), kc, g, r);
+					b[i] = load_kop<true, kRowLd>(d, 16 * (ot0 + i), kc, g, r);
+				}
+#pragma unroll
+				for (int i = 0; i < 2; ++i)
+#pragma unroll
+					for (int o2 = 0; o2 < 2; ++o2) accW[l][i][o2] = mfma(a[i], b[o2], accW[l][i][o2]);
+			}
+			scaled(&accW[l][0][0], 4, undo);
+		};
+		// this wave's loss sum, in a fixed order
+#pragma unroll
+		for (int off = 32; off >= 1; off >>= 1) lv += __shfl_xor(lv, off);
+		if (lane == 0) S.lsum[wave] += lv;
+
+		// ---- backward chain: delta_H = (W_H^T g_o) . 1[a_H > 0], then delta_l for l = H-1 .. 1
+		half8_t Bd[2];
+		{
+			float4_t acc[4];
+#pragma unroll
+			for (int mt = 0; mt < 4; ++mt) {
+				// W_H^T: K columns past the three outputs are zero (the block's rows 3..15 are)
+				const half8_t a = __builtin_shufflevector(tr_quad(H, 0, mt), (half4_t)0, 0, 1, 2, 3, 4, 5, 6, 7);
+				acc[mt] = mfma(a, Bg, (float4_t)0.0f);
+			}
+			const uint4 mH[2] = {act_masks(B[0]), act_masks(B[1])}; // B still holds a_H
+			relu_bwd_pack(acc, mH, Bd);
+			store_brow(S.dlt, Bd, g, col);
+		}
+		block_lds_sync(); // delta_H and the output gradients of every wave
+		// dW_H^T: input tile `wave` against the output-gradient rows
+		scaled(&accO, 1, dscale);
+#pragma unroll
+		for (int kc = 0; kc < R / 32; ++kc) {
+			const half8_t a = load_kop<true, kRowLd>(S.act[H], 16 * wave, kc, g, r);
+			const half8_t b = load_kop<false, kGoLd>(S.go, 0, kc, g, r);
+			accO = mfma(a, b, accO);
+		}
+		scaled(&accO, 1, undo);
+#pragma unroll
+		for (int l = H - 1; l >= 0; --l) {
+			// dW_l from a_l and delta_{l+1}, and delta_l from delta_{l+1}: independent
+			const bool in_dlt = ((H - 1 - l) & 1) == 0; // where delta_{l+1} lies
+			if (l >= 1) {
+				// the layer's eight W^T fragments are read from LDS together, so the
+				// MFMAs wait on one LDS round trip rather than on one each
+				half8_t wb[4][2];
+#pragma unroll
+				for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+					for (int mt = 0; mt < 4; ++mt) wb[mt][kc] = bwd_frag(l, mt, kc);
+				float4_t acc[4];
+#pragma unroll
+				for (int mt = 0; mt < 4; ++mt) acc[mt] = (float4_t)0.0f;
+#pragma unroll
+				for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+					for (int mt = 0; mt < 4; ++mt) acc[mt] = mfma(wb[mt][kc], Bd[kc], acc[mt]);
+				relu_bwd_pack(acc, keep[l], Bd);
+			}
+			dw_layer(l, in_dlt ? S.dlt : S.act[H]);
+			if (l >= 1) {
+				if (l == H - 1) block_lds_sync(); // the output layer's dW has read a_H, whose rows delta_{H-1} takes
+				store_brow(in_dlt ? S.act[H] : S.dlt, Bd, g, col);
+				block_lds_sync(); // delta_l of every wave
+			}
+		}
+	}
+	block_lds_sync(); // every wave's loss sum
+
+	// ---- the workgroup's partial row: dW tiles (float4 per lane) and the loss sum
+	store_row();
+	if (wave == 0 && lane == 0 && blk < gi.blocks) part[WC] = (S.lsum[0] + S.lsum[1]) + (S.lsum[2] + S.lsum[3]);
+	if (gi.overflow && __any(bad) && lane == 0) atomicOr(gi.overflow, 1u);
+}
+
 // N-tiles each wave runs through the layers together (1 or 2; both measure the
 // same, and 1 needs no register spill); VKNRC_INFER_TILES overrides.
 int infer_tiles() {
@@ -942,7 +1292,12 @@ template <int H, int ENC, bool F16IN> hipError_t infer_launch(const InferGroup &
 template <int H, int ENC, int LOSS, bool F16IN> hipError_t grad_small_attributes() {
 	static const hipError_t done = [] {
 		const int smem = (int)sizeof(SmallGradSmem<H>);
-		hipError_t e = hipFuncSetAttribute(
+		hipError_t e = hipSuccess;
+		if constexpr (!F16IN)
+			e = hipFuncSetAttribute(reinterpret_cast<const void *>(fused_grad_dual_kernel<H, ENC, LOSS>),
+			                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(DualGradSmem<H>));
+		if (e != hipSuccess) return e;
+		e = hipFuncSetAttribute(
 		    reinterpret_cast<const void *>(fused_grad_small_kernel<H, ENC, LOSS, F16IN, true>),
 		    hipFuncAttributeMaxDynamicSharedMemorySize, smem);
 		if (e == hipSuccess)
@@ -953,12 +1308,39 @@ template <int H, int ENC, int LOSS, bool F16IN> hipError_t grad_small_attributes
 	return done;
 }
 
-template <int H, int ENC, int LOSS, bool F16IN> hipError_t grad_small_launch(const GradGroup &grp, hipStream_t s) {
+// Sets block_begin and total_blocks and launches.
+template <int H, int ENC, int LOSS, bool F16IN> hipError_t grad_small_launch(GradGroup &grp, hipStream_t s) {
 	const size_t smem = sizeof(SmallGradSmem<H>);
 	bool multi = false;
-	for (uint32_t i = 0; i < grp.n_items; ++i) multi |= grp.item[i].chunks > 1;
+	uint32_t rows = 0, pairs = 0;
+	for (uint32_t i = 0; i < grp.n_items; ++i) {
+		multi |= grp.item[i].chunks > 1;
+		rows += grp.item[i].blocks;
+		pairs += (grp.item[i].blocks + 1) / 2;
+	}
+	// One row a CU (fused_grad_small_kernel), or two rows side by side (the same bits).  Rows
+	// run in rounds of one workgroup a CU, and a round of pairs takes 1.57 times a round of
+	// single rows (8 chunks a row: 67 us against 42.6), so the pairs win where they save more
+	// than that in rounds: 272 and 293 rows of 8 chunks 1.13x a 16-cache frame, 288 of 2 chunks
+	// 1.12x; not up to one row a CU, nor where both need a nearly empty last round (528 and 640
+	// rows: three rounds against two).  Rows of one chunk stay single: 512 to 1,984 of them
+	// took 0.95x a frame in pairs, which store all their sums at the end of a short row where
+	// the one-chunk kernel's stores drain during its backward.
+	const uint32_t cus = (uint32_t)device_cu_count();
+	const bool dual = !F16IN && multi && 8 * ((pairs + cus - 1) / cus) < 5 * ((rows + cus - 1) / cus);
+	grp.total_blocks = 0;
+	for (uint32_t i = 0; i < grp.n_items; ++i) {
+		grp.item[i].block_begin = grp.total_blocks;
+		grp.total_blocks += dual ? (grp.item[i].blocks + 1) / 2 : grp.item[i].blocks;
+	}
+	if (grp.total_blocks == 0) return hipSuccess;
 	hipError_t e = grad_small_attributes<H, ENC, LOSS, F16IN>();
 	if (e != hipSuccess) return e;
+	if constexpr (!F16IN)
+		if (dual) {
+			fused_grad_dual_kernel<H, ENC, LOSS><<<dim3(grp.total_blocks), dim3(512), sizeof(DualGradSmem<H>), s>>>(grp);
+			return hipGetLastError();
+		}
 	if (multi)
 		fused_grad_small_kernel<H, ENC, LOSS, F16IN, true><<<dim3(grp.total_blocks), dim3(256), smem, s>>>(grp);
 	else
@@ -971,12 +1353,12 @@ template <int H, int ENC> hipError_t prepare_enc(int loss) {
 	return grad_small_attributes<H, ENC, NRC_LOSS_RELATIVE_L2_LUMINANCE, false>();
 }
 
-template <int H, int ENC> hipError_t grad_group_enc(int loss, const GradGroup &g, hipStream_t s) {
+template <int H, int ENC> hipError_t grad_group_enc(int loss, GradGroup &g, hipStream_t s) {
 	if (loss == NRC_LOSS_L2) return grad_small_launch<H, ENC, NRC_LOSS_L2, false>(g, s);
 	return grad_small_launch<H, ENC, NRC_LOSS_RELATIVE_L2_LUMINANCE, false>(g, s);
 }
 
-template <int H> hipError_t grad_group_h(int encoding, int loss, const GradGroup &g, hipStream_t s) {
+template <int H> hipError_t grad_group_h(int encoding, int loss, GradGroup &g, hipStream_t s) {
 	switch (encoding) {
 	case NRC_ENCODING_TRI12: return grad_group_enc<H, NRC_ENCODING_TRI12>(loss, g, s);
 	case NRC_ENCODING_SINCOS6: return grad_group_enc<H, NRC_ENCODING_SINCOS6>(loss, g, s);
@@ -1084,13 +1466,6 @@ hipError_t prepare_fused(int hidden, int encoding, int loss) {
 }
 
 hipError_t launch_fused_gradient_group(int hidden, int encoding, int loss, GradGroup &grp, hipStream_t stream) {
-	uint32_t blocks = 0;
-	for (uint32_t i = 0; i < grp.n_items; ++i) {
-		grp.item[i].block_begin = blocks;
-		blocks += grp.item[i].blocks;
-	}
-	grp.total_blocks = blocks;
-	if (blocks == 0) return hipSuccess;
 	if (hidden == 5) return grad_group_h<5>(encoding, loss, grp, stream);
 	return grad_group_h<4>(encoding, loss, grp, stream);
 }
@@ -1138,7 +1513,6 @@ hipError_t launch_fused_gradient_f16(int hidden, const _Float16 *inputs, const f
 	it.chunks = p.chunks;
 	it.blocks = p.blocks;
 	it.pstride = pstride;
-	grp.total_blocks = p.blocks;
 	if (hidden == 5) return grad_small_launch<5, NRC_ENCODING_TRI12, NRC_LOSS_L2, true>(grp, stream);
 	return grad_small_launch<4, NRC_ENCODING_TRI12, NRC_LOSS_L2, true>(grp, stream);
 }
