@@ -75,6 +75,15 @@ __device__ __forceinline__ uint32_t effective_count(const uint32_t *d_count, uin
 	return c < clamp ? c : clamp;
 }
 
+// Workgroup barrier that orders LDS traffic only: the fences are restricted to
+// LDS, so the barrier waits on LDS counters and leaves global loads in flight
+// (for data exchanged through LDS; global memory needs __syncthreads).
+__device__ __forceinline__ void block_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+	__builtin_amdgcn_s_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Orders LDS traffic between lanes of one wavefront (LDS operations of a wave
 // execute in order; this keeps the compiler from moving them across).  The
 // fences are restricted to LDS so they wait on LDS counters only and leave the

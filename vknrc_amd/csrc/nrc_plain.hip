@@ -165,7 +165,7 @@ __device__ __forceinline__ void load_query(const float *__restrict__ q, float *r
 // nrc_inference.comp:30-48 (without the scene unpack and the epilogue).  Persistent, one
 // workgroup a CU, 16-record tiles dealt to the waves in turn.  Bound by the FP32 MFMA
 // rate: 336 MFMAs of 32 cycles a tile, 4.5 us of a SIMD.  230,400
-// queries: 203 -> 85 us (41 -> 112 TFLOP/s) against one thread a query on the vector unit.
+// queries: 203 -> 83.5 us (46 -> 114 TFLOP/s) against one thread a query on the vector unit.
 template <int H, int ENC>
 __global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const float *__restrict__ queries,
                                                                        const uint32_t *__restrict__ d_count,
@@ -173,17 +173,25 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const flo
                                                                        const float *__restrict__ w32,
                                                                        float *__restrict__ rgb) {
 	__shared__ PlainSmem<H> S;
-	stage_weights<H>(S, w32);
 	const uint32_t count = effective_count(d_count, max_count, max_count);
 	const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, slot = 16 * g + ((r + g) & 15);
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const uint32_t tiles = (count + 15) / 16;
-	for (uint32_t t = wave * gridDim.x + blockIdx.x; t < tiles; t += kPlainWaves * gridDim.x) {
-		const uint32_t n = t * 16 + r, last = count - 1;
-		float rec[kQueryFloats];
+	const uint32_t tiles = (count + 15) / 16, last = count - 1, stride = kPlainWaves * gridDim.x;
+	uint32_t t = wave * gridDim.x + blockIdx.x;
+	float rec[kQueryFloats];
+	// the first records are on their way while the weights are staged, the next ones while
+	// a tile runs (a tile past the last re-reads the last record)
+	auto load_tile = [&](uint32_t tile) __attribute__((always_inline)) {
+		const uint32_t n = tile < tiles ? tile * 16 + r : last;
 		load_query(queries + (size_t)(n < last ? n : last) * kQueryFloats, rec);
+	};
+	if (count > 0) load_tile(t); // uniform
+	stage_weights<H>(S, w32);
+	for (; t < tiles; t += stride) {
+		const uint32_t n = t * 16 + r;
 		float4_t x[4];
 		encode_lane<ENC>(rec, g, x);
+		load_tile(t + stride);
 #pragma unroll 1
 		for (int l = 0; l < H; ++l) layer_forward<H>(S, l, slot, x, x);
 		const float4_t o = output_forward<H>(S, lane, x);
@@ -198,7 +206,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const flo
 // (nrc_gradient.comp:26-58, NN_nv.glsl:162-278).  Writes the activations and deltas of a
 // tile as one 4 KB block [64 features][16 records] a layer, so that every store here and
 // every load of the reduction is a contiguous 256 or 1024 bytes a wave (rows of a whole
-// batch put each load on 16 lines 64 KB apart: the reduction took 25.7 us instead of 17.7).
+// batch put each load on 16 lines 64 KB apart: the reduction took 25.7 us instead of 17.7, before it went through LDS).
 // The records that pad the last tile are written as zeros, and the records of a tile are
 // stored in the order 4 (r & 3) + (r >> 2) that the reduction reads.  Bound by the FP32 MFMA rate
 // (592 of 32 cycles a tile for H = 5, 7.9 us of a SIMD; 16,384 records are one tile a
@@ -213,7 +221,6 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
                                                            float *__restrict__ acts, float *__restrict__ deltas,
                                                            float *__restrict__ sample_loss, uint32_t ldn) {
 	__shared__ PlainSmem<H> S;
-	stage_weights<H>(S, w32);
 	const uint32_t count = effective_count(d_count, max_count, clamp);
 	const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, slot = 16 * g + ((r + g) & 15);
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -227,13 +234,20 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 #pragma unroll
 	for (int i = 0; i < 4; ++i) tslot[i] = (16 * gp + ((4 * g + i + gp) & 15)) * 4 + (r & 3);
 	const float *sf = reinterpret_cast<const float *>(S.frag);
-	for (uint32_t t = wave * gridDim.x + blockIdx.x; t < tiles; t += kPlainWaves * gridDim.x) {
-		const uint32_t n = t * 16 + r, last = count - 1;
-		const bool valid = n < count;
-		const float *rp = records + (size_t)(valid ? n : last) * kTrainFloats;
-		float rec[kTrainFloats];
+	const uint32_t last = count - 1, stride = kPlainWaves * gridDim.x;
+	uint32_t t = wave * gridDim.x + blockIdx.x;
+	float rec[kTrainFloats];
+	auto load_tile = [&](uint32_t tile) __attribute__((always_inline)) {
+		const uint32_t n = tile < tiles ? tile * 16 + r : last;
+		const float *rp = records + (size_t)(n < last ? n : last) * kTrainFloats;
 #pragma unroll
 		for (int i = 0; i < kTrainFloats; ++i) rec[i] = rp[i];
+	};
+	if (count > 0) load_tile(t); // uniform; on their way while the weights are staged
+	stage_weights<H>(S, w32);
+	for (; t < tiles; t += stride) {
+		const uint32_t n = t * 16 + r;
+		const bool valid = n < count;
 		// features 16 mt + 4 i + g of this lane's record in the tile's block of a slab
 		const size_t blk = (size_t)t * (16 * kWidth) + 4 * (r & 3) + (r >> 2);
 		auto store = [&](float *dst, const float4_t *v) __attribute__((always_inline)) {
@@ -301,22 +315,24 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 				for (int i = 0; i < 4; ++i) d[m][i] = relu_bwd(acc[m][i], a[l][m][i]);
 			store(deltas + (size_t)(l - 1) * slab, d);
 		}
+		if (t + stride < tiles) load_tile(t + stride); // uniform
 	}
 }
 
 // Partial dW over one chunk of records: dW_l[m][k] = sum_n delta_l[m][n] a_l[k][n]
 // (NNUpdateDW64 / NNUpdateDW3, NN_nv.glsl:280-367), the records in order.  Grid: x over
-// half layers (32 output units) and the output layer, y over chunks; a wave computes two of
-// the 16x16 tiles as dW^T (A = activations, B = deltas, K = records, so a lane stores four
-// consecutive inputs), reading 16 bytes of a feature a lane straight from memory: in
-// the stored order a lane group's float4 holds records 4 j + g, the K index g of step j.
-// The loads of the next 64 records are in flight while the MFMAs of 64 run.  Also writes
-// the chunk's loss sum after the weights and flags non-finite partials.  Bound by the
-// reads of what the kernel before wrote (46 MB for 16,384 records, past the L2s) more than
-// by its MFMAs (256 a wave, 3.4 us).  16,384 records: 65 -> 17.7 us against
-// FMAs from LDS tiles.
+// the layers, y over chunks; wave w computes two of a layer's sixteen 16x16 tiles as dW^T (A =
+// activations, B = deltas, K = records, so a lane stores four consecutive inputs): in the
+// stored order a lane group's float4 holds records 4 j + g, the K index g of step j.  The 4 KB
+// blocks pass through LDS, two groups of 64 records ahead, so each is read once a layer and
+// chunk.  Also writes the chunk's loss sum after the weights and flags
+// non-finite partials.  Bound by the FP32 MFMA rate on the CUs that hold a workgroup (160
+// for 16,384 records: 512 MFMAs a SIMD, 6.8 us) and by the reads of what the kernel before
+// wrote (46 MB, past the L2s).  16,384 records: 65 us with FMAs from LDS tiles, 17.7 with
+// operands loaded by each wave for itself, 15.7 now.
+constexpr int kTiles = 4; // 16-record tiles a step
 template <int H>
-__global__ __launch_bounds__(256) void plain_dw_kernel(const uint32_t *__restrict__ d_count, uint32_t max_count,
+__global__ __launch_bounds__(512) void plain_dw_kernel(const uint32_t *__restrict__ d_count, uint32_t max_count,
                                                        uint32_t clamp, const float *__restrict__ acts,
                                                        const float *__restrict__ deltas,
                                                        const float *__restrict__ sample_loss, uint32_t ldn,
@@ -326,8 +342,7 @@ __global__ __launch_bounds__(256) void plain_dw_kernel(const uint32_t *__restric
 	const uint32_t count = effective_count(d_count, max_count, clamp);
 	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int g = lane >> 4, r = lane & 15;
-	const bool output = blockIdx.x == 2 * H;
-	const int l = (int)blockIdx.x >> 1; // H for the output layer
+	const int l = (int)blockIdx.x; // H: the output layer
 	const size_t slab = (size_t)kWidth * ldn;
 	const uint32_t nb0 = blockIdx.y * kPlainChunk;
 	uint32_t nend = nb0 + kPlainChunk;
@@ -339,58 +354,83 @@ __global__ __launch_bounds__(256) void plain_dw_kernel(const uint32_t *__restric
 #pragma unroll
 		for (int i = 0; i < 4; ++i) bad |= !isfinite(v[i]);
 	};
-	// NA input tiles from it0 against output tile ot (or, LAST, the three output rows)
-	auto tiles = [&](auto na, auto last, int it0, int ot) __attribute__((always_inline)) {
-		constexpr int NA = decltype(na)::value, STEPS = 4; // 16-record steps in flight
-		constexpr bool LAST = decltype(last)::value;
-		const bool live = !LAST || r < kOut;
-		const float *a = acts + (size_t)l * slab + 16 * (16 * it0 + r) + 4 * g;
-		const float *d = deltas + (size_t)l * slab + 16 * (16 * ot + (live ? r : 0)) + 4 * g;
-		float4_t acc[NA];
+	const uint32_t steps = nb0 < nend ? (nend - nb0 + 15) / 16 : 0; // 16-record tiles of this chunk
+	if (l < H) {
+		// kTiles tiles of a_l and delta_l are in LDS at a time, as they lie in memory; the next
+		// two groups are on their way through registers (direct copies to LDS would be waited
+		// for, all of them, before every read)
+		constexpr int kFloats = kTiles * 16 * kWidth, kPer = kFloats / 4 / 512, kGroups = (int)kPlainChunk / (16 * kTiles);
+		__shared__ __attribute__((aligned(16))) float buf[2][2][kFloats];
+		const float *src[2] = {acts + (size_t)l * slab + (size_t)nb0 * kWidth, deltas + (size_t)l * slab + (size_t)nb0 * kWidth};
+		const uint32_t words = steps * (16 * kWidth), tid = threadIdx.x;
+		float4_t next[2][2][kPer];
+		auto load = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll
-		for (int i = 0; i < NA; ++i) acc[i] = (float4_t)0.0f;
-		if (nb0 < nend) {
-			const uint32_t lastn = (nend - 1) & ~15u; // the last 16-record step
-			float4_t av[2][STEPS][NA], dv[2][STEPS];
-			auto load = [&](int b, uint32_t nb) __attribute__((always_inline)) {
+			for (int op = 0; op < 2; ++op)
 #pragma unroll
-				for (int k = 0; k < STEPS; ++k) {
-					const uint32_t n = nb + 16 * k < lastn ? nb + 16 * k : lastn;
-#pragma unroll
-					for (int i = 0; i < NA; ++i) av[b][k][i] = *reinterpret_cast<const float4_t *>(a + (size_t)n * kWidth + 256 * i);
-					dv[b][k] = *reinterpret_cast<const float4_t *>(d + (size_t)n * kWidth);
+				for (int k = 0; k < kPer; ++k) {
+					// past the chunk the loads repeat its last piece, which no step reads
+					const uint32_t w = (uint32_t)(grp * kFloats + k * 2048) + 4u * tid;
+					next[grp & 1][op][k] = *reinterpret_cast<const float4_t *>(src[op] + (w < words ? w : words - 4u));
 				}
-			};
-			auto run = [&](int b, uint32_t nb) __attribute__((always_inline)) {
+		};
+		auto store = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll
-				for (int k = 0; k < STEPS; ++k)
-					if (nb + 16 * k < nend) // uniform
+			for (int op = 0; op < 2; ++op)
 #pragma unroll
-						for (int j = 0; j < 4; ++j)
-#pragma unroll
-							for (int i = 0; i < NA; ++i) acc[i] = mfma4(av[b][k][i][j], live ? dv[b][k][j] : 0.0f, acc[i]);
-			};
-			load(0, nb0);
-			for (uint32_t nb = nb0; nb < nend; nb += 32 * STEPS) {
-				load(1, nb + 16 * STEPS);
-				run(0, nb);
-				load(0, nb + 32 * STEPS);
-				run(1, nb + 16 * STEPS);
-			}
+				for (int k = 0; k < kPer; ++k) *reinterpret_cast<float4_t *>(&buf[grp & 1][op][k * 2048 + 4u * tid]) = next[grp & 1][op][k];
+		};
+		const int it0 = 2 * (wave & 1), ot = wave >> 1;
+		float4_t acc[2] = {(float4_t)0.0f, (float4_t)0.0f};
+		if (steps > 0) {
+			load(0);
+			load(1);
+			store(0);
 		}
-		if (live)
 #pragma unroll
-			for (int i = 0; i < NA; ++i) put(pp + l * kWidth * kWidth + (16 * ot + r) * kWidth + 16 * (it0 + i) + 4 * g, acc[i]);
-	};
-	if (!output) {
-		tiles(std::integral_constant<int, 2>{}, std::false_type{}, 2 * (wave & 1), 2 * ((int)blockIdx.x & 1) + (wave >> 1));
+		for (int grp = 0; grp < kGroups; ++grp) {
+			if ((uint32_t)(grp * kTiles) >= steps) break; // uniform
+			load(grp + 2);
+			block_lds_sync();
+			const float4_t *pa = reinterpret_cast<const float4_t *>(buf[grp & 1][0]) + (16 * it0 + r) * 4 + g;
+			const float4_t *pd = reinterpret_cast<const float4_t *>(buf[grp & 1][1]) + (16 * ot + r) * 4 + g;
+#pragma unroll
+			for (int k = 0; k < kTiles; ++k) {
+				if ((uint32_t)(grp * kTiles + k) >= steps) break; // uniform
+				const float4_t a0 = pa[k * 256], a1 = pa[k * 256 + 64], d = pd[k * 256];
+#pragma unroll
+				for (int e = 0; e < 4; ++e) {
+					acc[0] = mfma4(a0[e], d[e], acc[0]);
+					acc[1] = mfma4(a1[e], d[e], acc[1]);
+				}
+			}
+			store(grp + 1); // into the buffer that the group before this one was read from
+		}
+#pragma unroll
+		for (int i = 0; i < 2; ++i) put(pp + l * kWidth * kWidth + (16 * ot + r) * kWidth + 16 * (it0 + i) + 4 * g, acc[i]);
 	} else {
-		tiles(std::integral_constant<int, 1>{}, std::true_type{}, wave, 0);
+		// the output layer: wave w < 4 computes input tile w against the three output rows
+		if (wave < 4) {
+			const bool live = r < kOut;
+			const float *a = acts + (size_t)H * slab + (size_t)nb0 * kWidth + 16 * (16 * wave + r) + 4 * g;
+			const float *d = deltas + (size_t)H * slab + (size_t)nb0 * kWidth + 16 * (live ? r : 0) + 4 * g;
+			float4_t acc = (float4_t)0.0f;
+#pragma unroll 8
+			for (uint32_t k = 0; k < steps; ++k) {
+				const float4_t av = *reinterpret_cast<const float4_t *>(a + (size_t)k * (16 * kWidth));
+				const float4_t dv = *reinterpret_cast<const float4_t *>(d + (size_t)k * (16 * kWidth));
+#pragma unroll
+				for (int e = 0; e < 4; ++e) acc = mfma4(av[e], live ? dv[e] : 0.0f, acc);
+			}
+			if (live) put(pp + H * kWidth * kWidth + r * kWidth + 16 * wave + 4 * g, acc);
+		}
 		__shared__ float sl[256];
 		const int t = threadIdx.x;
 		float v = 0.0f;
-		for (uint32_t n = nb0 + t; n < nend; n += 256) v += sample_loss[n];
-		sl[t] = v;
+		if (t < 256) {
+			for (uint32_t n = nb0 + t; n < nend; n += 256) v += sample_loss[n];
+			sl[t] = v;
+		}
 		__syncthreads();
 		for (int s = 128; s > 0; s >>= 1) {
 			if (t < s) sl[t] += sl[t + s];
@@ -459,7 +499,7 @@ template <int H> void plain_gradient_h(const TrainArgs &a, uint32_t nparts, hipS
 	case NRC_ENCODING_SINCOS6: plain_fwdbwd_loss<H, NRC_ENCODING_SINCOS6>(a, s); break;
 	default: plain_fwdbwd_loss<H, NRC_ENCODING_UV_SINCOS16>(a, s); break;
 	}
-	const dim3 grid(2 * H + 1, nparts), block(256);
+	const dim3 grid(H + 1, nparts), block(512);
 	plain_dw_kernel<H><<<grid, block, 0, s>>>(a.d_count, a.max_count, a.clamp, a.acts, a.deltas, a.sample_loss, a.ldn,
 	                                          a.partials, a.pstride, &a.state->overflow[a.parity]);
 }
