@@ -81,8 +81,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	oneblob_sel8_init(sSel[wave], lane);
 	const int h = lane >> 5, r = lane & 31;
-	const uint32_t t0 = (uint32_t)((uint64_t)grp.total_tiles * blockIdx.x / gridDim.x);
-	const uint32_t t1 = (uint32_t)((uint64_t)grp.total_tiles * (blockIdx.x + 1) / gridDim.x);
+	const uint32_t tiles = infer_tiles(grp);
+	const uint32_t t0 = (uint32_t)((uint64_t)tiles * blockIdx.x / gridDim.x);
+	const uint32_t t1 = (uint32_t)((uint64_t)tiles * (blockIdx.x + 1) / gridDim.x);
 	uint32_t *const slot = sX[wave];
 	const Fp8SlotEmit emit{slot, h, r, sSel[wave]}; // this lane encodes record r of N-tile h
 

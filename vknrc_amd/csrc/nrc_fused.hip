@@ -39,8 +39,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 	wave_lds_sync();
 	const int g = lane >> 4, r = lane & 15;
 	const uint32_t nW = gridDim.x * 4, gw = blockIdx.x * 4 + wave;
-	const uint32_t t0 = (uint32_t)((uint64_t)grp.total_tiles * gw / nW);
-	const uint32_t t1 = (uint32_t)((uint64_t)grp.total_tiles * (gw + 1) / nW);
+	const uint32_t tiles = infer_tiles(grp);
+	const uint32_t t0 = (uint32_t)((uint64_t)tiles * gw / nW);
+	const uint32_t t1 = (uint32_t)((uint64_t)tiles * (gw + 1) / nW);
 	half8_t *sx = sX[wave];
 	half4_t *sx4 = reinterpret_cast<half4_t *>(sx);
 	const int et = lane >> 4, es = lane & 15; // this lane's record: tile et, column es
@@ -240,8 +241,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 	wave_lds_sync();
 	const int g = lane >> 4, r = lane & 15;
 	const uint32_t nW = gridDim.x * 4, gw = blockIdx.x * 4 + wave;
-	const uint32_t t0 = (uint32_t)((uint64_t)grp.total_tiles * gw / nW);
-	const uint32_t t1 = (uint32_t)((uint64_t)grp.total_tiles * (gw + 1) / nW);
+	const uint32_t tiles = infer_tiles(grp);
+	const uint32_t t0 = (uint32_t)((uint64_t)tiles * gw / nW);
+	const uint32_t t1 = (uint32_t)((uint64_t)tiles * (gw + 1) / nW);
 	half8_t *slot0 = sX0[wave], *slot1 = sX1[wave];
 	const int et = lane >> 4, es = lane & 15; // this lane's record: N-tile et, column es
 	// the output clamp max(o, 0) as a signed integer max of the bits: every value with
@@ -1254,7 +1256,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // N-tiles each wave runs through the layers together (1 or 2; both measure the
 // same, and 1 needs no register spill); VKNRC_INFER_TILES overrides.
-int infer_tiles() {
+int infer_tiles_override() {
 	static const int t = [] {
 		const char *e = getenv("VKNRC_INFER_TILES");
 		return (e && atoi(e) == 2) ? 2 : 1;
@@ -1280,7 +1282,7 @@ template <int H, int ENC, bool F16IN> hipError_t infer_launch(const InferGroup &
 	if (blocks == 0) blocks = 1;
 	if (!F16IN && infer_pipelined())
 		fused_infer_pipe_kernel<H, ENC><<<dim3(blocks), dim3(256), 0, s>>>(grp);
-	else if (infer_tiles() == 1)
+	else if (infer_tiles_override() == 1)
 		fused_infer_kernel<H, ENC, F16IN, 1><<<dim3(blocks), dim3(256), 0, s>>>(grp);
 	else
 		fused_infer_kernel<H, ENC, F16IN, 2><<<dim3(blocks), dim3(256), 0, s>>>(grp);

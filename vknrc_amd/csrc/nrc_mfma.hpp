@@ -50,6 +50,17 @@ __device__ __forceinline__ half8_t pack_relu(float4_t lo, float4_t hi) {
 	return h;
 }
 
+// The tiles that an inference launch deals to its waves.  One cache: those of the records
+// that there are (the device count), so that a count below the maximum leaves no wave
+// without work (700,001 of 921,600 queries: 36.1 us dealt by the maximum, 33.0 by the
+// count).  Several: those of the maxima, which the host has added up; the counts of all of
+// them would have to be fetched one after the other first.
+__device__ __forceinline__ uint32_t infer_tiles(const InferGroup &grp) {
+	if (grp.n_items != 1) return grp.total_tiles;
+	const InferItem &it = grp.item[0];
+	return (__builtin_amdgcn_readfirstlane(effective_count(it.d_count, it.max_count, it.max_count)) + 63u) / 64u;
+}
+
 // Calls f(std::integral_constant<int, i>{}) for i = 0 .. N-1, unrolled at compile time.
 template <typename F, int... I> __device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
 	(f(std::integral_constant<int, I>{}), ...);
