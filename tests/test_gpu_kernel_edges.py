@@ -169,11 +169,12 @@ def test_fp8_inference_tiles(hidden, enc):
         assert (y[live:] == 7.0).all()
 
 
-# the unpack takes 64 records a wave through LDS, four lanes fetching one record's scene data:
+# a launch for many records takes a wave's 64 through LDS, one for few goes straight to memory:
 # every lane of a partial wave, one wave and one record more, a device count inside a wave, odd
 # record addresses; each prefix gives the rows of the whole, and nothing past the count is written
+@pytest.mark.parametrize("room", [0, 70000])
 @pytest.mark.parametrize("packed", [False, True])
-def test_unpack_partial_waves(packed):
+def test_unpack_partial_waves(packed, room):
     s = wl.make_scene(5, primitives=300, vertices=200, instances=3, materials=5, textures=2, texture_size=16)
     ds = v.DeviceScene(torch, s["vertices"], s["vertex_indices"], s["texcoords"], s["texcoord_indices"], s["materials"],
                        s["material_ids"], s["transforms"], s["textures"])
@@ -188,8 +189,10 @@ def test_unpack_partial_waves(packed):
     words = lambda a: dev(np.concatenate([np.zeros(1, np.int32), np.frombuffer(a.tobytes(), np.int32)]))[1:]  # noqa: E731
 
     def rows(fn, rec, width, n, live):
+        rec = np.concatenate([rec[:n], np.zeros(max(room - n, 0), rec.dtype)])
+        n = len(rec)
         out = torch.full((n, width), 7.0, device=DEV)
-        fn(ds, words(rec[:n]), n, out, count=dev(np.array([live], np.uint32).view(np.int32)))
+        fn(ds, words(rec), n, out, count=dev(np.array([live], np.uint32).view(np.int32)))
         y = host(out)
         assert (y[live:] == 7.0).all()
         return y[:live]

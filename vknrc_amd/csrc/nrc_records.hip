@@ -50,67 +50,57 @@ __device__ __forceinline__ void repeat_texels(float u, uint32_t n, uint32_t &i0,
 }
 
 // texture(sampler2D, uv).rgb with linear filtering and repeat addressing
-// (NRCRenderGraph.cpp:132) of an RGBA8 sRGB image (VkScene.cpp:193)
-__device__ void sample_texture(const nrc_texture &t, float u, float v, const float *lut, float *o) {
-	uint32_t x0, x1, y0, y1;
+// (NRCRenderGraph.cpp:132) of an RGBA8 sRGB image (VkScene.cpp:193), in two halves so that the
+// texels of both of a material's textures are on their way together: fetch() issues the loads,
+// color() blends.  GetSceneDiffuse / GetSceneSpecular (Scene.glsl:63-68): an id past the
+// texture table, or an empty texture, takes the constant colour.
+struct TexelFetch {
+	uint32_t p00, p01, p10, p11;
 	float ax, ay;
-	repeat_texels(u, t.width, x0, x1, ax);
-	repeat_texels(v, t.height, y0, y1, ay);
-	const uint32_t p00 = t.d_rgba8[(size_t)y0 * t.width + x0], p01 = t.d_rgba8[(size_t)y0 * t.width + x1];
-	const uint32_t p10 = t.d_rgba8[(size_t)y1 * t.width + x0], p11 = t.d_rgba8[(size_t)y1 * t.width + x1];
-#pragma unroll
-	for (int c = 0; c < 3; ++c) {
-		const uint32_t sh = 8u * (uint32_t)c;
-		const float c00 = lut[(p00 >> sh) & 255u], c01 = lut[(p01 >> sh) & 255u];
-		const float c10 = lut[(p10 >> sh) & 255u], c11 = lut[(p11 >> sh) & 255u];
-		const float top = c00 + ax * (c01 - c00), bot = c10 + ax * (c11 - c10);
-		o[c] = top + ay * (bot - top);
-	}
-}
+	bool textured;
 
-// GetSceneDiffuse / GetSceneSpecular (Scene.glsl:63-68); an id past the texture
-// table, or an empty texture, takes the constant colour
-__device__ __forceinline__ void material_color(const nrc_scene &s, const float *constant, uint32_t tex, float u, float v,
-                                               const float *lut, float *o) {
-	const nrc_texture *t = (tex == kNoTexture || s.d_textures == nullptr || tex >= s.texture_count) ? nullptr
-	                                                                                               : s.d_textures + tex;
-	if (t == nullptr || t->width == 0u || t->height == 0u || t->d_rgba8 == nullptr) {
-		o[0] = constant[0];
-		o[1] = constant[1];
-		o[2] = constant[2];
-	} else {
-		sample_texture(*t, u, v, lut, o);
+	__device__ __forceinline__ void fetch(const nrc_texture &t, bool valid, float u, float v) {
+		textured = valid && t.width != 0u && t.height != 0u && t.d_rgba8 != nullptr;
+		p00 = p01 = p10 = p11 = 0u;
+		ax = ay = 0.0f;
+		if (textured) {
+			uint32_t x0, x1, y0, y1;
+			repeat_texels(u, t.width, x0, x1, ax);
+			repeat_texels(v, t.height, y0, y1, ay);
+			p00 = t.d_rgba8[(size_t)y0 * t.width + x0];
+			p01 = t.d_rgba8[(size_t)y0 * t.width + x1];
+			p10 = t.d_rgba8[(size_t)y1 * t.width + x0];
+			p11 = t.d_rgba8[(size_t)y1 * t.width + x1];
+		}
 	}
+	__device__ __forceinline__ void color(const float *constant, const float *lut, float *o) const {
+		if (!textured) {
+			o[0] = constant[0];
+			o[1] = constant[1];
+			o[2] = constant[2];
+			return;
+		}
+#pragma unroll
+		for (int c = 0; c < 3; ++c) {
+			const uint32_t sh = 8u * (uint32_t)c;
+			const float c00 = lut[(p00 >> sh) & 255u], c01 = lut[(p01 >> sh) & 255u];
+			const float c10 = lut[(p10 >> sh) & 255u], c11 = lut[(p11 >> sh) & 255u];
+			const float top = c00 + ax * (c01 - c00), bot = c10 + ax * (c11 - c10);
+			o[c] = top + ay * (bot - top);
+		}
+	}
+};
+
+__device__ __forceinline__ bool texture_id_valid(const nrc_scene &s, uint32_t tex) {
+	return tex != kNoTexture && s.d_textures != nullptr && tex < s.texture_count;
 }
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef f4v __attribute__((aligned(4))) f4v_any;
 
-// The 16-byte pieces 0 .. PIECES-1 of record `index` of this lane, from 64 lanes' records of
-// `stride` bytes at any 4-byte alignment.  Four neighbouring lanes fetch one record, so a
-// load instruction touches 16 lines instead of 64 (the vector cache looks up a line or so a
-// cycle, which bounds these gathers), and the pieces go to their lanes through the wave's
-// 4 KB of LDS, pieces rotated by lane so that neither side conflicts on banks.  Every lane
-// of the wave takes part; a lane without a record passes some valid index.
-template <int PIECES>
-__device__ __forceinline__ void gather_records(const void *base, uint32_t stride, uint32_t index, int lane, f4v *buf, f4v *out) {
-	const int piece = lane & 3;
-	f4v v[4];
-#pragma unroll
-	for (int k = 0; k < 4; ++k) {
-		const uint32_t i = (uint32_t)__shfl((int)index, 16 * k + (lane >> 2));
-		if (piece < PIECES)
-			v[k] = *reinterpret_cast<const f4v_any *>(static_cast<const char *>(base) + (size_t)i * stride + 16 * piece);
-	}
-#pragma unroll
-	for (int k = 0; k < 4; ++k) {
-		const int rec = 16 * k + (lane >> 2);
-		if (piece < PIECES) buf[rec * 4 + (piece ^ ((rec >> 2) & 3))] = v[k];
-	}
-	wave_lds_sync();
-#pragma unroll
-	for (int j = 0; j < PIECES; ++j) out[j] = buf[lane * 4 + (j ^ ((lane >> 2) & 3))];
-	wave_lds_sync();
+// Piece j of a record of 16-byte pieces at any 4-byte alignment
+__device__ __forceinline__ f4v record_piece(const void *record, int j) {
+	return *reinterpret_cast<const f4v_any *>(static_cast<const char *>(record) + 16 * j);
 }
 
 // A primitive's corners (object space), their texture coordinates and its material:
@@ -135,9 +125,9 @@ __device__ __forceinline__ PrimitiveData indexed_primitive(const nrc_scene &s, u
 	return d;
 }
 
-__device__ __forceinline__ PrimitiveData packed_primitive(const f4v *r) {
+__device__ __forceinline__ PrimitiveData packed_primitive(const nrc_scene_primitive *r) {
 	PrimitiveData d;
-	const f4v a = r[0], b = r[1], c = r[2], e = r[3];
+	const f4v a = record_piece(r, 0), b = record_piece(r, 1), c = record_piece(r, 2), e = record_piece(r, 3);
 	d.c[0][0] = a[0]; d.c[0][1] = a[1]; d.c[0][2] = a[2];
 	d.c[1][0] = a[3]; d.c[1][1] = b[0]; d.c[1][2] = b[1];
 	d.c[2][0] = b[2]; d.c[2][1] = b[3]; d.c[2][2] = c[0];
@@ -155,20 +145,17 @@ __device__ __forceinline__ void transform_vertex(const float *T, const float *v,
 	for (int j = 0; j < 3; ++j) o[j] = T[4 * j] * v[0] + T[4 * j + 1] * v[1] + T[4 * j + 2] * v[2] + T[4 * j + 3];
 }
 
-// UnpackNRCInput (NRCRecord.glsl:98-125) into the 14 floats of an nrc_query; `buf` is the
-// wave's 4 KB of LDS, and every lane of the wave calls this
+// UnpackNRCInput (NRCRecord.glsl:98-125) into the 14 floats of an nrc_query
 template <bool PACKED>
-__device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, const float *lut, int lane, f4v *buf, float *q) {
+__device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, const float *lut, float *q) {
 	const uint32_t prim = p.primitive_id, inst = p.flip_bit_instance_id & 0x7FFFFFFFu;
 	const bool flip = (p.flip_bit_instance_id >> 31) != 0u;
+	f4v rows[3];
+#pragma unroll
+	for (int j = 0; j < 3; ++j) rows[j] = record_piece(s.d_transforms + (size_t)inst * 12, j);
 	PrimitiveData d;
-	if constexpr (PACKED) {
-		f4v r[4];
-		gather_records<4>(s.d_primitives, 64u, prim, lane, buf, r);
-		d = packed_primitive(r);
-	} else {
-		d = indexed_primitive(s, prim);
-	}
+	if constexpr (PACKED) d = packed_primitive(s.d_primitives + prim);
+	else d = indexed_primitive(s, prim);
 	// opaque values, so that the compiler fuses the products below into the sums in the same
 	// way whichever way they were loaded: the packed records give the bits of the index arrays
 #pragma unroll
@@ -176,9 +163,27 @@ __device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, cons
 		asm volatile("" : "+v"(d.c[k][0]), "+v"(d.c[k][1]), "+v"(d.c[k][2]));
 		asm volatile("" : "+v"(d.t[k][0]), "+v"(d.t[k][1]));
 	}
-	f4v rows[3], mat[4];
-	gather_records<3>(s.d_transforms, 48u, inst, lane, buf, rows);
-	gather_records<4>(s.d_materials, 64u, d.material, lane, buf, mat);
+	const nrc_material *m = s.d_materials + d.material;
+	const f4v mat[2] = {record_piece(m, 0), record_piece(m, 1)};
+	const float roughness = m->roughness;
+	const float diffuse[3] = {mat[0][0], mat[0][1], mat[0][2]}, specular[3] = {mat[1][0], mat[1][1], mat[1][2]};
+	const float dt = mat[0][3], st = mat[1][3];
+	const uint32_t tex[2] = {__float_as_uint(dt), __float_as_uint(st)};
+	nrc_texture t[2] = {};
+	bool valid[2];
+#pragma unroll
+	for (int k = 0; k < 2; ++k) {
+		valid[k] = texture_id_valid(s, tex[k]);
+		if (valid[k]) t[k] = s.d_textures[tex[k]];
+	}
+	float b[3];
+	unorm2x16(p.barycentric_2x16u, b + 1);
+	b[0] = 1.0f - b[1] - b[2];
+	const float u = d.t[0][0] * b[0] + d.t[1][0] * b[1] + d.t[2][0] * b[2];
+	const float v = d.t[0][1] * b[0] + d.t[1][1] * b[1] + d.t[2][1] * b[2];
+	TexelFetch texels[2];
+#pragma unroll
+	for (int k = 0; k < 2; ++k) texels[k].fetch(t[k], valid[k], u, v);
 	const float T[12] = {rows[0][0], rows[0][1], rows[0][2], rows[0][3], rows[1][0], rows[1][1],
 	                     rows[1][2], rows[1][3], rows[2][0], rows[2][1], rows[2][2], rows[2][3]};
 	float v0[3], v1[3], v2[3];
@@ -193,24 +198,16 @@ __device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, cons
 	n[0] *= sgn;
 	n[1] *= sgn;
 	n[2] *= sgn;
-	float b[3];
-	unorm2x16(p.barycentric_2x16u, b + 1);
-	b[0] = 1.0f - b[1] - b[2];
 #pragma unroll
 	for (int j = 0; j < 3; ++j) q[j] = v0[j] * b[0] + v1[j] * b[1] + v2[j] * b[2];
 	unorm2x16(p.scattered_dir_2x16u, q + 3);
 	sph_encode(n[0], n[1], n[2], q + 5);
-	const float diffuse[3] = {mat[0][0], mat[0][1], mat[0][2]}, specular[3] = {mat[1][0], mat[1][1], mat[1][2]};
-	const float dt = mat[0][3], st = mat[1][3];
-	q[7] = mat[3][1]; // roughness
-	const float u = d.t[0][0] * b[0] + d.t[1][0] * b[1] + d.t[2][0] * b[2];
-	const float v = d.t[0][1] * b[0] + d.t[1][1] * b[1] + d.t[2][1] * b[2];
-	material_color(s, diffuse, __float_as_uint(dt), u, v, lut, q + 8);
-	material_color(s, specular, __float_as_uint(st), u, v, lut, q + 11);
+	q[7] = roughness;
+	texels[0].color(diffuse, lut, q + 8);
+	texels[1].color(specular, lut, q + 11);
 }
 static_assert(offsetof(nrc_material, diffuse_texture_id) == 12 && offsetof(nrc_material, specular) == 16 &&
-                  offsetof(nrc_material, specular_texture_id) == 28 && offsetof(nrc_material, roughness) == 52 &&
-                  sizeof(nrc_material) == 64,
+                  offsetof(nrc_material, specular_texture_id) == 28,
               "the material fields that unpack_input picks from 16-byte pieces");
 
 __device__ __forceinline__ nrc_packed_input load_packed(const uint32_t *w) {
@@ -224,47 +221,66 @@ __device__ __forceinline__ nrc_packed_input load_packed(const uint32_t *w) {
 
 // Unpacks wire records of WORDS dwords, whose packed input starts at dword AT, into rows of
 // FLOATS floats (queries, or training records with the record's bias as the target,
-// nrc_gradient.comp:30-33).  A wave's 64 records come in and its rows go out through its LDS
-// as contiguous dwords (any 4-byte alignment), where a record a lane straight from and to
-// memory touched 10 to 56 lines an instruction.  Bound by the vector cache's line look-ups
-// (8 a record, 14.5 without the shared gathers), the vector unit (690 instructions a
-// record) and the misses of L2 (1.3 a record), each busy for about 60 % of the time.
-// 2,073,600 eval records on random packed primitives: 80.3 -> 67 us.
+// nrc_gradient.comp:30-33), a record a lane.  STAGED: a wave's 64 records come in and its rows
+// go out through its LDS as contiguous dwords (any 4-byte alignment), where a record straight
+// from and to memory touches 10 to 56 lines an instruction.  Bound by the vector cache's line
+// look-ups, the vector unit (690 instructions a record) and the misses of L2 (1.3 a record),
+// each busy for over half of the time; the chain record, primitive, material, texture, texels
+// has the next record's loads to hide behind in a large launch only, so what does not depend
+// on each other is loaded together (both textures before the geometry is worked out).
+// Random packed primitives: 2,073,600 eval records 80 -> 64 us, 65,536 train records
+// 7.0 -> 5.8 us; indexed primitives 151 -> 141 and 9.6 -> 9.2 us.
 constexpr uint32_t kUnpackWaves = 4;
-template <bool PACKED, int WORDS, int AT, int FLOATS>
+template <bool PACKED, bool STAGED, int WORDS, int AT, int FLOATS>
 __global__ __launch_bounds__(64 * kUnpackWaves) void unpack_kernel(const nrc_scene s, const uint32_t *__restrict__ rec,
                                                      const uint32_t *d_count, uint32_t max_count,
                                                      float *__restrict__ out) {
 	__shared__ float lut[256];
-	constexpr int kWaveWords = 64 * (FLOATS > 16 ? FLOATS : 16); // records in, then gathers, then rows out
-	__shared__ __attribute__((aligned(16))) uint32_t stage[kUnpackWaves][kWaveWords];
-	static_assert(WORDS <= 16, "the records fit the stage");
-	srgb_table_init(lut);
+	constexpr int kWaveWords = STAGED ? 64 * (FLOATS > WORDS ? FLOATS : WORDS) : 1; // records in, then rows out
+	__shared__ uint32_t stage[kUnpackWaves][kWaveWords];
 	const uint32_t count = effective_count(d_count, max_count, max_count);
 	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	uint32_t *const st = stage[wave];
 	const uint32_t first = (blockIdx.x * kUnpackWaves + (uint32_t)wave) * 64u;
-	if (first >= count) return; // uniform over the wave
-	const uint32_t n = count - first < 64u ? count - first : 64u;
+	const uint32_t n = first >= count ? 0u : count - first < 64u ? count - first : 64u;
 	const uint32_t *src = rec + (size_t)first * WORDS;
+	uint32_t w[WORDS]; // on their way while the table is built
+	if constexpr (STAGED) {
 #pragma unroll
-	for (int k = 0; k < WORDS; ++k)
-		if (lane + 64u * k < n * WORDS) st[lane + 64u * k] = src[lane + 64u * k];
-	wave_lds_sync();
-	const uint32_t *w = st + ((uint32_t)lane < n ? (uint32_t)lane : n - 1u) * WORDS; // a lane past the count repeats the last record
-	const nrc_packed_input p = load_packed(w + AT);
+		for (int k = 0; k < WORDS; ++k) w[k] = lane + 64u * k < n * WORDS ? src[lane + 64u * k] : 0u;
+	} else {
+#pragma unroll
+		for (int k = 0; k < WORDS; ++k) w[k] = (uint32_t)lane < n ? src[lane * WORDS + k] : 0u;
+	}
+	srgb_table_init(lut);
+	if (STAGED) {
+		if (n == 0u) return; // uniform over the wave
+#pragma unroll
+		for (int k = 0; k < WORDS; ++k) st[lane + 64u * k] = w[k];
+		wave_lds_sync();
+		const uint32_t at = ((uint32_t)lane < n ? (uint32_t)lane : n - 1u) * WORDS; // a lane past the count repeats the last record
+#pragma unroll
+		for (int k = 0; k < WORDS; ++k) w[k] = st[at + k];
+		wave_lds_sync();
+	} else if ((uint32_t)lane >= n) {
+		return;
+	}
 	float q[FLOATS];
+	unpack_input<PACKED>(s, load_packed(w + AT), lut, q);
 #pragma unroll
 	for (int k = kQueryFloats; k < FLOATS; ++k) q[k] = __uint_as_float(w[k - kQueryFloats]);
-	wave_lds_sync();
-	unpack_input<PACKED>(s, p, lut, lane, reinterpret_cast<f4v *>(st), q);
+	float *dst = out + (size_t)first * FLOATS;
+	if constexpr (STAGED) {
 #pragma unroll
-	for (int k = 0; k < FLOATS; ++k) st[lane * FLOATS + k] = __float_as_uint(q[k]);
-	wave_lds_sync();
-	uint32_t *dst = reinterpret_cast<uint32_t *>(out) + (size_t)first * FLOATS;
+		for (int k = 0; k < FLOATS; ++k) st[lane * FLOATS + k] = __float_as_uint(q[k]);
+		wave_lds_sync();
 #pragma unroll
-	for (int k = 0; k < FLOATS; ++k)
-		if (lane + 64u * k < n * FLOATS) dst[lane + 64u * k] = st[lane + 64u * k];
+		for (int k = 0; k < FLOATS; ++k)
+			if (lane + 64u * k < n * FLOATS) dst[lane + 64u * k] = __uint_as_float(st[lane + 64u * k]);
+	} else {
+#pragma unroll
+		for (int k = 0; k < FLOATS; ++k) dst[lane * FLOATS + k] = q[k];
+	}
 }
 
 // One thread per primitive: the corners and texture coordinates its indices name and
@@ -430,10 +446,17 @@ hipError_t launch_unpack(const nrc_scene &s, const void *rec, const uint32_t *d_
 	if (max_count == 0) return hipSuccess;
 	const dim3 grid((max_count + 64u * kUnpackWaves - 1u) / (64u * kUnpackWaves)), block(64 * kUnpackWaves);
 	const uint32_t *r = static_cast<const uint32_t *>(rec);
+	// Up to half a wave a SIMD (32,768 records) nothing hides the two passes through LDS, and the
+	// vector cache has look-ups to spare.  Straight and staged: 4,096 train records 5.14 and
+	// 5.64 us on packed primitives, 5.9 and 6.4 on indexed ones; 16,384 eval records 5.25 and
+	// 5.31, 6.0 and 6.5; 65,536 train records 6.37 and 6.30; 230,400 eval records 12.4 and 11.4.
+	const bool staged = (uint64_t)grid.x * kUnpackWaves > 2u * (uint64_t)device_cu_count();
 	if (s.d_primitives)
-		unpack_kernel<true, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out);
+		staged ? unpack_kernel<true, true, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out)
+		       : unpack_kernel<true, false, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out);
 	else
-		unpack_kernel<false, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out);
+		staged ? unpack_kernel<false, true, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out)
+		       : unpack_kernel<false, false, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out);
 	return hipGetLastError();
 }
 static_assert(sizeof(nrc_eval_record) == 20 && sizeof(nrc_wire_train_record) == 40, "wire records in dwords");
