@@ -67,6 +67,23 @@ def test_mlp_gradient_reduction_edges(hidden, n):
     assert rel_err(host(dw), G) < GRAD_F16_TOL
 
 
+# more streams than kept scratch blocks, in flight together: each call has a block of its own
+# or one ordered behind its last use, so the bits are those of the calls one at a time
+def test_mlp_gradient_streams():
+    rng = np.random.default_rng(11)
+    w = dev(rng.normal(0, np.sqrt(2 / 64), v.weight_count(5)).astype(np.float16))
+    x, t = dev(rng.uniform(-1, 1, (12 * 4096, 64)).astype(np.float16)), dev(rng.uniform(0, 1, (12 * 4096, 3)).astype(np.float32))
+    calls = [(x[4096 * k:4096 * (k + 1)], t[4096 * k:4096 * (k + 1)]) for k in range(12)]
+    one, many = (torch.zeros((12, v.weight_count(5)), device=DEV) for _ in range(2))
+    for k, (xk, tk) in enumerate(calls):
+        v.mlp_gradient_f16(w, xk, tk, 4096, one[k])
+        torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    for k, (xk, tk) in enumerate(calls):
+        v.mlp_gradient_f16(w, xk, tk, 4096, many[k], stream=streams[k % 4])
+    assert np.array_equal(host(many), host(one))
+
+
 # the forward gathers row-major weights with wide loads where their address allows it and
 # single halves where it does not: the same fragments, so the same bits
 @pytest.mark.parametrize("hidden", [4, 5])

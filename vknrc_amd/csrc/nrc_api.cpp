@@ -261,12 +261,13 @@ nrc_status check_train(nrc_cache *c, const nrc_train_record *d_records, uint32_t
 
 // Scratch of the stateless gradient (nrc_mlp_gradient_f16): a few blocks per GPU kept
 // between calls, each guarded by the event of its last use.  A call takes a block that no
-// other host thread holds, makes its stream wait for that event (on whatever stream it was
-// recorded) and records the event again after its last kernel, so calls on several streams
-// and threads never share a block in use.  With no block free, or under stream capture,
-// the scratch is stream-ordered as a library's is (hipMallocAsync, hipFreeAsync).  Those
-// two cost 25-40 us of host time a call: a forward and a gradient of 16,384 rows took
-// 109 us a pass with them, 33 us of it in kernels (38 us a pass with a kept block).
+// other host thread holds and that its own stream used last, or whose last use is over; it
+// makes its stream wait for that event and records the event again after its last kernel, so
+// calls on several streams and threads never share a block in use, nor wait for each other.
+// With no such block, or under stream capture, the scratch is stream-ordered as a library's
+// is (hipMallocAsync, hipFreeAsync).  Those two cost 25-40 us of host time a call: a forward
+// and a gradient of 16,384 rows took 109 us a pass with them, 33 us of it in kernels (38 us
+// a pass with a kept block).
 constexpr int kMaxDevices = 64, kScratchBlocks = 2;
 // one gradient workgroup a CU writes one row: 256 rows and both fragment copies, 21.3 MB
 constexpr size_t kScratchBytes = 2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDEN_LAYERS) + nrc::bwd_frag_halves(NRC_MAX_HIDDEN_LAYERS)) +
@@ -274,6 +275,7 @@ constexpr size_t kScratchBytes = 2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDE
 struct ScratchBlock {
 	void *p = nullptr;
 	hipEvent_t done = nullptr;
+	hipStream_t last = nullptr; // compared only: a reused handle still waits for `done`
 	bool held = false;
 };
 std::mutex g_scratch_mu;
@@ -283,6 +285,24 @@ struct Scratch {
 	void *p = nullptr;
 	ScratchBlock *block = nullptr; // null: stream-ordered
 
+	static ScratchBlock *find(ScratchBlock (&blocks)[kScratchBlocks], hipStream_t s) {
+		for (ScratchBlock &b : blocks)
+			if (b.p && !b.held && b.last == s) return &b;
+		for (ScratchBlock &b : blocks) {
+			if (b.held) continue;
+			if (b.p) {
+				if (hipEventQuery(b.done) == hipSuccess) return &b;
+				continue;
+			}
+			if (hipEventCreateWithFlags(&b.done, hipEventDisableTiming) != hipSuccess) return nullptr;
+			if (hipMalloc(&b.p, kScratchBytes) == hipSuccess) return &b;
+			(void)hipEventDestroy(b.done);
+			b = ScratchBlock{};
+			return nullptr;
+		}
+		return nullptr;
+	}
+
 	hipError_t take(size_t bytes, hipStream_t s) {
 		int dev = 0;
 		hipError_t e = hipGetDevice(&dev);
@@ -291,26 +311,18 @@ struct Scratch {
 		const bool captured = hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 		if (!captured && bytes <= kScratchBytes && dev >= 0 && dev < kMaxDevices) {
 			std::lock_guard<std::mutex> lock(g_scratch_mu);
-			for (ScratchBlock &b : g_scratch[dev]) {
-				if (b.held) continue;
-				if (!b.p) {
-					hipEvent_t done = nullptr;
-					void *q = nullptr;
-					if (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) break;
-					if (hipMalloc(&q, kScratchBytes) != hipSuccess) {
-						(void)hipEventDestroy(done);
-						break;
-					}
-					b.p = q;
-					b.done = done;
-				} else if (hipStreamWaitEvent(s, b.done, 0) != hipSuccess) {
-					break;
-				}
-				b.held = true;
-				block = &b;
-				p = b.p;
+			// relaxed: a capture that another stream has under way neither forbids nor sees
+			// the allocation and the queries
+			hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+			const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+			block = find(g_scratch[dev], s);
+			if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+			if (block && hipStreamWaitEvent(s, block->done, 0) == hipSuccess) {
+				block->held = true;
+				p = block->p;
 				return hipSuccess;
 			}
+			block = nullptr;
 		}
 		(void)hipGetLastError();
 		return hipMallocAsync(&p, bytes, s);
@@ -321,6 +333,7 @@ struct Scratch {
 		if (!block) return hipFreeAsync(p, s);
 		std::lock_guard<std::mutex> lock(g_scratch_mu);
 		const hipError_t e = hipEventRecord(block->done, s);
+		block->last = s;
 		if (e == hipSuccess) block->held = false; // a block whose use cannot be marked is never handed out again
 		return e;
 	}
