@@ -30,7 +30,8 @@ namespace {
 
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kPlainWaves = 8; // waves of a workgroup; one workgroup a CU (its LDS holds the FP32 weights)
+// waves of a workgroup; one workgroup a CU (its LDS holds the FP32 weights)
+constexpr int kPlainWaves = 8, kPlainInferWaves = 16;
 
 __device__ __forceinline__ float4_t mfma4(float a, float b, float4_t c) {
 	return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -42,13 +43,13 @@ template <int H> struct PlainSmem {
 };
 
 // All weights into LDS, every load in flight before the first store.
-template <int H> __device__ __forceinline__ void stage_weights(PlainSmem<H> &S, const float *__restrict__ w32) {
-	constexpr int kPer = H * 1024 / (64 * kPlainWaves);
+template <int H, int WAVES> __device__ __forceinline__ void stage_weights(PlainSmem<H> &S, const float *__restrict__ w32) {
+	constexpr int kPer = H * 1024 / (64 * WAVES);
 	const int t = threadIdx.x;
 	const float4_t *src = reinterpret_cast<const float4_t *>(w32);
 	float4_t v[kPer];
 #pragma unroll
-	for (int k = 0; k < kPer; ++k) v[k] = src[t + k * 64 * kPlainWaves];
+	for (int k = 0; k < kPer; ++k) v[k] = src[t + k * 64 * WAVES];
 	if (t < 4 * 64) {
 		const int mt = t >> 6, g = (t >> 4) & 3, r = t & 15;
 		const float *wo = w32 + H * kWidth * kWidth + (r < kOut ? r : 0) * kWidth + 16 * mt + g;
@@ -59,7 +60,7 @@ template <int H> __device__ __forceinline__ void stage_weights(PlainSmem<H> &S, 
 #pragma unroll
 	for (int k = 0; k < kPer; ++k) {
 		// layer j >> 10, row (j >> 4) & 63, columns 16 mt + 4 i + 0..3
-		const int j = t + k * 64 * kPlainWaves, row = (j >> 4) & 63, mt = (j >> 2) & 3, i = j & 3;
+		const int j = t + k * 64 * WAVES, row = (j >> 4) & 63, mt = (j >> 2) & 3, i = j & 3;
 		const int r = 4 * (row & 3) + ((row >> 2) & 3), blk = ((j >> 10) * 4 + (row >> 4)) * 4 + mt;
 #pragma unroll
 		for (int g = 0; g < 4; ++g) f[(blk * 64 + 16 * g + ((r + g) & 15)) * 4 + i] = v[k][g];
@@ -164,10 +165,14 @@ __device__ __forceinline__ void load_query(const float *__restrict__ q, float *r
 
 // nrc_inference.comp:30-48 (without the scene unpack and the epilogue).  Persistent, one
 // workgroup a CU, 16-record tiles dealt to the waves in turn.  Bound by the FP32 MFMA
-// rate: 336 MFMAs of 32 cycles a tile, 4.5 us of a SIMD.  230,400
-// queries: 203 -> 83.5 us (46 -> 114 TFLOP/s) against one thread a query on the vector unit.
+// rate, 336 MFMAs of 32 cycles a tile, plus the 270 (TRI12) vector instructions of a tile:
+// FP32 MFMAs and vector instructions never overlap (no co-issued cycle counted), 4.9 us of a
+// SIMD together.  Four waves a SIMD fill the waits that two left (87.3 -> 84.3 us for
+// 230,400 queries back to back, 681 -> 660 us for 2,073,600); fragments read a step ahead
+// add nothing to that.  230,400 queries: 203 -> 81.0 us against one thread a query on the
+// vector unit.
 template <int H, int ENC>
-__global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const float *__restrict__ queries,
+__global__ __launch_bounds__(64 * kPlainInferWaves) void plain_infer_kernel(const float *__restrict__ queries,
                                                                        const uint32_t *__restrict__ d_count,
                                                                        uint32_t max_count,
                                                                        const float *__restrict__ w32,
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const flo
 	const uint32_t count = effective_count(d_count, max_count, max_count);
 	const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, slot = 16 * g + ((r + g) & 15);
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-	const uint32_t tiles = (count + 15) / 16, last = count - 1, stride = kPlainWaves * gridDim.x;
+	const uint32_t tiles = (count + 15) / 16, last = count - 1, stride = kPlainInferWaves * gridDim.x;
 	uint32_t t = wave * gridDim.x + blockIdx.x;
 	float rec[kQueryFloats];
 	// the first records are on their way while the weights are staged, the next ones while
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const flo
 		load_query(queries + (size_t)(n < last ? n : last) * kQueryFloats, rec);
 	};
 	if (count > 0) load_tile(t); // uniform
-	stage_weights<H>(S, w32);
+	stage_weights<H, kPlainInferWaves>(S, w32);
 	for (; t < tiles; t += stride) {
 		const uint32_t n = t * 16 + r;
 		float4_t x[4];
@@ -206,13 +211,13 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_infer_kernel(const flo
 // (nrc_gradient.comp:26-58, NN_nv.glsl:162-278).  Writes the activations and deltas of a
 // tile as one 4 KB block [64 features][16 records] a layer, so that every store here and
 // every load of the reduction is a contiguous 256 or 1024 bytes a wave (rows of a whole
-// batch put each load on 16 lines 64 KB apart: the reduction took 25.7 us instead of 17.7, before it went through LDS).
-// The records that pad the last tile are written as zeros, and the records of a tile are
-// stored in the order 4 (r & 3) + (r >> 2) that the reduction reads.  Bound by the FP32 MFMA rate
-// (592 of 32 cycles a tile for H = 5, 7.9 us of a SIMD; 16,384 records are one tile a
-// SIMD) and the 46 MB of activations and deltas written.
-// 16,384 records: 397 -> 25.7 us against one thread a record (64 workgroups on 256 CUs,
-// a broadcast LDS read a product).
+// batch put each load on 16 lines 64 KB apart: the reduction took 25.7 us instead of 17.7,
+// before it went through LDS).  The records that pad the last tile are written as zeros, and
+// the records of a tile are stored in the order 4 (r & 3) + (r >> 2) that the reduction
+// reads.  Bound by the FP32 MFMA rate (592 of 32 cycles a tile for H = 5, 7.9 us of a SIMD;
+// 16,384 records are one tile a SIMD), the 46 MB of activations and deltas written and the
+// staging of the weights before the first tile.  16,384 records: 397 -> 25.2 us against one
+// thread a record (64 workgroups on 256 CUs, a broadcast LDS read a product).
 template <int H, int ENC, int LOSS>
 __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const float *__restrict__ records,
                                                            const uint32_t *__restrict__ d_count, uint32_t max_count,
@@ -244,7 +249,7 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 		for (int i = 0; i < kTrainFloats; ++i) rec[i] = rp[i];
 	};
 	if (count > 0) load_tile(t); // uniform; on their way while the weights are staged
-	stage_weights<H>(S, w32);
+	stage_weights<H, kPlainWaves>(S, w32);
 	for (; t < tiles; t += stride) {
 		const uint32_t n = t * 16 + r;
 		const bool valid = n < count;
@@ -473,7 +478,7 @@ uint32_t plain_blocks(uint32_t n) {
 template <int H>
 hipError_t plain_infer_h(int enc, const float *q, const uint32_t *dc, uint32_t mc, const float *w, float *rgb,
                          hipStream_t s) {
-	const dim3 grid(plain_blocks(mc)), block(64 * kPlainWaves);
+	const dim3 grid(plain_blocks(mc)), block(64 * kPlainInferWaves);
 	switch (enc) {
 	case NRC_ENCODING_TRI12: plain_infer_kernel<H, NRC_ENCODING_TRI12><<<grid, block, 0, s>>>(q, dc, mc, w, rgb); break;
 	case NRC_ENCODING_SINCOS6: plain_infer_kernel<H, NRC_ENCODING_SINCOS6><<<grid, block, 0, s>>>(q, dc, mc, w, rgb); break;
