@@ -121,24 +121,36 @@ template <int ENC> __device__ __forceinline__ void encode_lane(const float *rec,
 	}
 }
 
-// y = relu(W_l x) of this wave's 16 records (NN_nv.glsl:99-127); four independent
-// accumulator chains, one 16-byte LDS read per four MFMAs
-template <int H> __device__ __forceinline__ void layer_forward(const PlainSmem<H> &S, int l, int slot, const float4_t *x, float4_t *y) {
+// The A fragments of layer l that the K steps 4 mt .. 4 mt + 3 take
+template <int H> __device__ __forceinline__ void layer_fragments(const PlainSmem<H> &S, int l, int mt, int slot, float4_t *a) {
+#pragma unroll
+	for (int m = 0; m < 4; ++m) a[m] = S.frag[((l * 4 + m) * 4 + mt) * 64 + slot];
+}
+
+// x = relu(W_l x) of this wave's 16 records (NN_nv.glsl:99-127); four independent
+// accumulator chains, one 16-byte LDS read per four MFMAs.  `next` holds the layer's first
+// fragments and receives those of the layer after it (the first layer's after the last): a
+// wave that has its SIMD to itself would otherwise wait for each read.
+template <int H> __device__ __forceinline__ void layer_forward(const PlainSmem<H> &S, int l, int slot, float4_t *x, float4_t *next) {
 	float4_t acc[4];
 #pragma unroll
 	for (int m = 0; m < 4; ++m) acc[m] = (float4_t)0.0f;
+	const int after = l + 1 < H ? l + 1 : 0;
 #pragma unroll
 	for (int mt = 0; mt < 4; ++mt) {
 		float4_t a[4];
 #pragma unroll
-		for (int m = 0; m < 4; ++m) a[m] = S.frag[((l * 4 + m) * 4 + mt) * 64 + slot];
+		for (int m = 0; m < 4; ++m) a[m] = next[m];
+		layer_fragments<H>(S, mt < 3 ? l : after, (mt + 1) & 3, slot, next);
+		__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
 		for (int i = 0; i < 4; ++i)
 #pragma unroll
 			for (int m = 0; m < 4; ++m) acc[m] = mfma4(a[m][i], x[mt][i], acc[m]);
+		__builtin_amdgcn_sched_barrier(0);
 	}
 #pragma unroll
-	for (int m = 0; m < 4; ++m) y[m] = relu4(acc[m]);
+	for (int m = 0; m < 4; ++m) x[m] = relu4(acc[m]);
 }
 
 // o = W_H x (NN_nv.glsl:129-158), padded to 16 rows: lane group 0 holds the outputs
@@ -168,9 +180,8 @@ __device__ __forceinline__ void load_query(const float *__restrict__ q, float *r
 // rate, 336 MFMAs of 32 cycles a tile, plus the 270 (TRI12) vector instructions of a tile:
 // FP32 MFMAs and vector instructions never overlap (no co-issued cycle counted), 4.9 us of a
 // SIMD together.  Four waves a SIMD fill the waits that two left (87.3 -> 84.3 us for
-// 230,400 queries back to back, 681 -> 660 us for 2,073,600); fragments read a step ahead
-// add nothing to that.  230,400 queries: 203 -> 81.0 us against one thread a query on the
-// vector unit.
+// 230,400 queries back to back, 681 -> 660 us for 2,073,600; 655 with the fragments read
+// ahead).  230,400 queries: 203 -> 80.3 us against one thread a query on the vector unit.
 template <int H, int ENC>
 __global__ __launch_bounds__(64 * kPlainInferWaves) void plain_infer_kernel(const float *__restrict__ queries,
                                                                        const uint32_t *__restrict__ d_count,
@@ -192,13 +203,15 @@ __global__ __launch_bounds__(64 * kPlainInferWaves) void plain_infer_kernel(cons
 	};
 	if (count > 0) load_tile(t); // uniform
 	stage_weights<H, kPlainInferWaves>(S, w32);
+	float4_t next[4];
+	layer_fragments<H>(S, 0, 0, slot, next);
 	for (; t < tiles; t += stride) {
 		const uint32_t n = t * 16 + r;
 		float4_t x[4];
 		encode_lane<ENC>(rec, g, x);
 		load_tile(t + stride);
 #pragma unroll 1
-		for (int l = 0; l < H; ++l) layer_forward<H>(S, l, slot, x, x);
+		for (int l = 0; l < H; ++l) layer_forward<H>(S, l, slot, x, next);
 		const float4_t o = output_forward<H>(S, lane, x);
 		if (g == 0 && n < count)
 #pragma unroll
@@ -216,8 +229,10 @@ __global__ __launch_bounds__(64 * kPlainInferWaves) void plain_infer_kernel(cons
 // the records of a tile are stored in the order 4 (r & 3) + (r >> 2) that the reduction
 // reads.  Bound by the FP32 MFMA rate (592 of 32 cycles a tile for H = 5, 7.9 us of a SIMD;
 // 16,384 records are one tile a SIMD), the 46 MB of activations and deltas written and the
-// staging of the weights before the first tile.  16,384 records: 397 -> 25.2 us against one
-// thread a record (64 workgroups on 256 CUs, a broadcast LDS read a product).
+// staging of the weights before the first tile.  16,384 records: 397 -> 25.8 us against one
+// thread a record (64 workgroups on 256 CUs, a broadcast LDS read a product), 23.2 with the
+// layers as loops and the weights read ahead; 4.4 of that are the launch and the staging,
+// 2 to 3 the stores (non-temporal stores move as much to the reduction).
 template <int H, int ENC, int LOSS>
 __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const float *__restrict__ records,
                                                            const uint32_t *__restrict__ d_count, uint32_t max_count,
@@ -250,6 +265,8 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 	};
 	if (count > 0) load_tile(t); // uniform; on their way while the weights are staged
 	stage_weights<H, kPlainWaves>(S, w32);
+	float4_t next[4];
+	layer_fragments<H>(S, 0, 0, slot, next);
 	for (; t < tiles; t += stride) {
 		const uint32_t n = t * 16 + r;
 		const bool valid = n < count;
@@ -261,19 +278,35 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 #pragma unroll
 				for (int i = 0; i < 4; ++i) dst[blk + 16 * (16 * mt + 4 * i + g)] = v[mt][i];
 		};
-		float4_t a[H + 1][4];
-		encode_lane<ENC>(rec, g, a[0]);
+		float4_t x[4];
+		encode_lane<ENC>(rec, g, x);
 #pragma unroll
 		for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-			for (int i = 0; i < 4; ++i) a[0][mt][i] = valid ? a[0][mt][i] : 0.0f;
-		store(acts, a[0]);
-#pragma unroll
+			for (int i = 0; i < 4; ++i) x[mt][i] = valid ? x[mt][i] : 0.0f;
+		store(acts, x);
+		// 1[a_l > 0] of this lane's units, 16 bits a layer, the latest layer lowest.  With the
+		// bits instead of the activations in registers the layers are loops, whose code is
+		// fetched once: a launch is one tile a wave, and its first pass over 25 KB of unrolled
+		// layers waited for the instructions.
+		uint32_t active[3] = {0u, 0u, 0u};
+		static_assert(H <= 6, "16 H bits in three words");
+#pragma unroll 1
 		for (int l = 0; l < H; ++l) {
-			layer_forward<H>(S, l, slot, a[l], a[l + 1]);
-			store(acts + (size_t)(l + 1) * slab, a[l + 1]);
+			layer_forward<H>(S, l, slot, x, next);
+			store(acts + (size_t)(l + 1) * slab, x);
+			active[2] = __builtin_amdgcn_alignbit(active[2], active[1], 16);
+			active[1] = __builtin_amdgcn_alignbit(active[1], active[0], 16);
+			active[0] <<= 16;
+#pragma unroll
+			for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+				for (int i = 0; i < 4; ++i) active[0] |= (x[mt][i] > 0.0f ? 1u : 0u) << (4 * mt + i);
 		}
-		const float4_t ov = output_forward<H>(S, lane, a[H]);
+		auto relu_mask = [&active](float v, int unit) __attribute__((always_inline)) {
+			return relu_bwd(v, (active[0] >> unit) & 1u ? 1.0f : 0.0f);
+		};
+		const float4_t ov = output_forward<H>(S, lane, x);
 		const float o[kOut] = {__shfl(ov[0], r), __shfl(ov[1], r), __shfl(ov[2], r)}; // from lane group 0
 		float go[kOut];
 		const float v = loss_grad<LOSS>(o, rec + kQueryFloats, s, go);
@@ -297,27 +330,41 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 				float y = w0[i] * go[0];
 				y = fmaf(w1[i], go[1], y);
 				y = fmaf(w2[i], go[2], y);
-				d[mt][i] = relu_bwd(y, a[H][mt][i]);
+				d[mt][i] = relu_mask(y, 4 * mt + i);
 			}
 		}
 		store(deltas + (size_t)(H - 1) * slab, d);
 		// delta_{l-1} = (W_l^T delta_l) . 1[a_l > 0], l = H-1..1  (NNBackwardDA64_ReLU, NN_nv.glsl:248-278)
-#pragma unroll
+#pragma unroll 1
 		for (int l = H - 1; l >= 1; --l) {
+			active[0] = __builtin_amdgcn_alignbit(active[1], active[0], 16);
+			active[1] = __builtin_amdgcn_alignbit(active[2], active[1], 16);
+			active[2] >>= 16;
 			float4_t acc[4];
-#pragma unroll
-			for (int m = 0; m < 4; ++m) acc[m] = (float4_t)0.0f;
-#pragma unroll
-			for (int mt = 0; mt < 4; ++mt)
+			float w[2][4][4]; // the weights of four K steps, read while the four before them run
+			auto read = [&](int mt) __attribute__((always_inline)) {
 #pragma unroll
 				for (int i = 0; i < 4; ++i)
 #pragma unroll
-					for (int m = 0; m < 4; ++m)
-						acc[m] = mfma4(sf[((l * 4 + mt) * 4 + m) * 256 + tslot[i]], d[mt][i], acc[m]);
+					for (int m = 0; m < 4; ++m) w[mt & 1][i][m] = sf[((l * 4 + mt) * 4 + m) * 256 + tslot[i]];
+			};
+#pragma unroll
+			for (int m = 0; m < 4; ++m) acc[m] = (float4_t)0.0f;
+			read(0);
+#pragma unroll
+			for (int mt = 0; mt < 4; ++mt) {
+				if (mt < 3) read(mt + 1);
+				__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+				for (int i = 0; i < 4; ++i)
+#pragma unroll
+					for (int m = 0; m < 4; ++m) acc[m] = mfma4(w[mt & 1][i][m], d[mt][i], acc[m]);
+				__builtin_amdgcn_sched_barrier(0);
+			}
 #pragma unroll
 			for (int m = 0; m < 4; ++m)
 #pragma unroll
-				for (int i = 0; i < 4; ++i) d[m][i] = relu_bwd(acc[m][i], a[l][m][i]);
+				for (int i = 0; i < 4; ++i) d[m][i] = relu_mask(acc[m][i], 4 * m + i);
 			store(deltas + (size_t)(l - 1) * slab, d);
 		}
 		if (t + stride < tiles) load_tile(t + stride); // uniform
