@@ -261,19 +261,21 @@ def test_gradient_row_pairs(hidden, enc, loss):
         e["cache"].close()
 
 
-# one cache's inference deals the tiles of the device count: counts around a tile, far below the
-# maximum and zero give the rows of the whole and write nothing past the count
+# one cache's inference deals the tiles of the device count if there are more than waves (2,048), else
+# those of the maximum: counts around a tile, far below the maximum and zero give the rows of the whole
+# and write nothing past the count
+@pytest.mark.parametrize("n", [70001, 140001])
 @pytest.mark.parametrize("hidden,enc", ENCODINGS)
-def test_f16_inference_deals_the_counted_tiles(hidden, enc):
-    w, r = plain_inputs(hidden, enc, 70001)
+def test_f16_inference_deals_the_counted_tiles(hidden, enc, n):
+    w, r = plain_inputs(hidden, enc, n)
     st = v.NRCState(v.NRCConfig(hidden_layers=hidden, encoding=enc))
     st.set_state(weight=w)
     q = dev(r[:, :14])
-    whole = torch.zeros((70001, 3), device=DEV)
+    whole = torch.zeros((n, 3), device=DEV)
     st.infer(q, whole)
     whole = host(whole)
-    for live in (0, 1, 63, 64, 65, 2048 * 64 // 4 + 1, 70000):
-        out = torch.full((70001, 3), 7.0, device=DEV)
+    for live in (0, 1, 63, 64, 65, 2048 * 64 // 4 + 1, n - 1):
+        out = torch.full((n, 3), 7.0, device=DEV)
         st.infer(q, out, count=dev(np.array([live], np.uint32).view(np.int32)))
         y = host(out)
         assert np.array_equal(y[:live], whole[:live]), live
