@@ -262,18 +262,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void f
 
 __device__ __forceinline__ float pow2_floor(float x) { return ldexpf(1.0f, ilogbf(x)); }
 
+// The maximum over the 16 lanes of a row, in each of them (rotations by 8, 4, 2 and 1)
+__device__ __forceinline__ float row_max(float x) {
+	auto with = [](float v, auto ctrl) __attribute__((always_inline)) {
+		const int o = __builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), decltype(ctrl)::value, 0xF, 0xF, false);
+		return fmaxf(v, __uint_as_float((uint32_t)o));
+	};
+	x = with(x, std::integral_constant<int, 0x128>{}); // row_ror:8
+	x = with(x, std::integral_constant<int, 0x124>{});
+	x = with(x, std::integral_constant<int, 0x122>{});
+	return with(x, std::integral_constant<int, 0x121>{});
+}
+
 // One block per cache: folds the last FP8 inference's per-block maxima into the history,
 // chooses the layer scales and writes the e4m3 copy of c_l W_l.  Bound by latency: the
-// maxima, the history and the weights (held in registers, five float4 a thread) are all
-// loaded before anything waits; one kernel of 1,024 threads takes 8.3 us where a scale
-// kernel of 256 and a quantize kernel took 8.5 + 4.8 us and a launch.
+// maxima, the history, the scales and the weights (held in registers, five float4 a thread)
+// are all loaded before anything waits, the barriers do not wait for the stores (nothing in
+// this kernel reads them), and the maxima go over rows of lanes and then a wave each.
+// 6.3 us; 8.2 with full barriers, shuffles over whole waves and one thread a maximum; a
+// scale kernel of 256 threads and a quantize kernel took 8.5 + 4.8 us and a launch.
 template <int H> __global__ __launch_bounds__(1024) void fp8_prep_kernel(const Fp8PrepGroup grp) {
 	static_assert(kFp8MaxBlocks == 1024, "one slot of the last inference's maxima a thread");
 	const Fp8PrepItem &it = grp.item[blockIdx.x];
 	Fp8State *st = it.f8;
 	const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-	__shared__ float red[2 * kFp8Layers][16]; // wave maxima: activations, then |W_l|
-	__shared__ float hist_old[kFp8History][kFp8Layers], cscale[kFp8Layers];
+	__shared__ float red[2 * kFp8Layers][64]; // maxima of 16 threads: activations, then |W_l|
+	__shared__ float largest[2 * kFp8Layers], hist_old[kFp8History][kFp8Layers], cscale[kFp8Layers];
+	static_assert(kFp8History == 16 && 2 * kFp8Layers <= 16, "a row of lanes for the history, a wave for each maximum");
 
 	// 1. every load: the last inference's activation maxima (scaled by its C_l), the history, the weights
 	float m[2 * kFp8Layers];
@@ -281,6 +296,7 @@ template <int H> __global__ __launch_bounds__(1024) void fp8_prep_kernel(const F
 	for (int l = 0; l < kFp8Layers; ++l) m[l] = st->block_amax[t][l];
 	const uint32_t frames0 = st->frames;
 	const bool recorded = st->scale[0] > 0.0f; // a previous call set the scales that inference used
+	const float scale_old = st->scale[wave < kFp8Layers ? wave : 0];
 	const float hv = t < kFp8History * kFp8Layers ? (&st->hist[0][0])[t] : 0.0f;
 	const float4_t *w4 = reinterpret_cast<const float4_t *>(it.use32);
 	float4_t w[H + 1];
@@ -298,55 +314,55 @@ template <int H> __global__ __launch_bounds__(1024) void fp8_prep_kernel(const F
 		                           : 0.0f;
 #pragma unroll
 	for (int k = 0; k < 2 * kFp8Layers; ++k) {
-#pragma unroll
-		for (int off = 32; off >= 1; off >>= 1) m[k] = fmaxf(m[k], __shfl_xor(m[k], off));
-		if (lane == 0) red[k][wave] = m[k];
+		m[k] = row_max(m[k]);
+		if ((lane & 15) == 0) red[k][t >> 4] = m[k];
 	}
 	if (t < kFp8History * kFp8Layers) (&hist_old[0][0])[t] = hv;
-	__syncthreads();
+	block_lds_sync();
 
-	// 3. thread l < H: the history maximum of layer l + 1's input; threads kFp8Layers + l: |W_l|
-	if (t < 2 * kFp8Layers) {
-		float mx = red[t][0];
-#pragma unroll
-		for (int j = 1; j < 16; ++j) mx = fmaxf(mx, red[t][j]);
-		if (t < kFp8Layers) {
+	// 3. wave l <= H: the history maximum of layer l's input; waves kFp8Layers + l: |W_l|
+	if (wave < 2 * kFp8Layers) {
+		float mx = row_max(red[wave][lane]);
+		mx = fmaxf(mx, __shfl_xor(mx, 16));
+		mx = fmaxf(mx, __shfl_xor(mx, 32));
+		if (wave < kFp8Layers) {
 			uint32_t frames = frames0;
-			if (recorded && t <= H) {
+			float past = hist_old[lane & 15][wave];
+			if (recorded && wave <= H) {
 				const uint32_t slot = frames % kFp8History;
-				const float v = t == 0 ? 1.0f : mx / st->scale[t];
-				st->hist[slot][t] = v;
-				hist_old[slot][t] = v;
+				const float v = wave == 0 ? 1.0f : mx / scale_old;
+				if (lane == 0) st->hist[slot][wave] = v;
+				if ((uint32_t)(lane & 15) == slot) past = v;
 				++frames;
 			}
 			const uint32_t nh = frames < (uint32_t)kFp8History ? frames : (uint32_t)kFp8History;
-			mx = 0.0f;
-			for (uint32_t k = 0; k < nh; ++k) mx = fmaxf(mx, hist_old[k][t]);
+			mx = fmaxf(row_max((uint32_t)(lane & 15) < nh ? past : 0.0f), 0.0f);
 			if (nh == 0) mx = 4.0f; // no history yet: a first guess, corrected after one inference
-			if (t == 0 && recorded) st->frames = frames;
 		}
-		red[t][0] = mx;
+		if (lane == 0) largest[wave] = mx;
 	}
-	__syncthreads();
-	// the scales: c_l for l < H from the history, c_H from the weights
+	block_lds_sync();
+	// the scales: c_l for l < H from the history, c_H from the weights (every wave has its
+	// copy of what this overwrites)
 	if (t == 0) {
+		if (recorded) st->frames = frames0 + 1u;
 		float C = 1.0f;
 		st->scale[0] = 1.0f;
 #pragma unroll
 		for (int l = 0; l < H; ++l) {
-			const float hmax = red[l + 1][0], wmax = red[kFp8Layers + l][0];
+			const float hmax = largest[l + 1], wmax = largest[kFp8Layers + l];
 			float c = (hmax > 0.0f) ? pow2_floor(kFp8Target / (hmax * C)) : 1.0f;
 			if (wmax > 0.0f && wmax * c > kFp8Max) c = pow2_floor(kFp8Max / wmax);
 			st->wscale[l] = cscale[l] = c;
 			C *= c;
 			st->scale[l + 1] = C;
 		}
-		const float wmax = red[kFp8Layers + H][0];
+		const float wmax = largest[kFp8Layers + H];
 		const float cH = wmax > 0.0f ? pow2_floor(kFp8Max / wmax) : 1.0f;
 		st->wscale[H] = cscale[H] = cH;
 		st->out_scale = 1.0f / (cH * C);
 	}
-	__syncthreads();
+	block_lds_sync();
 
 	// 4. the e4m3 copy: four weights of a row are four consecutive bytes of a fragment
 #pragma unroll
