@@ -156,3 +156,52 @@ def test_two_knot_exact_cases():
             if 0 <= pos < 4:
                 want[i, pos] = v
     assert np.array_equal(got, want)
+
+
+# ---- the e4m3 quad of the FP8 inference (oneblob4_fp8): one byte permute with kOneBlobSel8
+
+
+def e4m3(x):
+    from oracle.fp8 import e4m3_round
+    return e4m3_round(x)
+
+
+def fp8_quad(x):
+    """oneblob4_fp8: the knots at j - 4x and (j + 1) - 4x, placed by the selector of med3(j, -2, 5), which is
+    -2 for a NaN (the median of a NaN and two numbers is their minimum); the four e4m3 values."""
+    src = re.search(r"kOneBlobSel8\[8\]\s*=\s*\{(.*?)\};", open(HEADER).read(), re.S).group(1)
+    tab = [int(v, 16) for v in re.findall(r"0x([0-9A-Fa-f]+)u", src)]
+    assert len(tab) == 8
+    with np.errstate(all="ignore"):
+        x4 = (F32(4) * x).astype(F32)
+        j = np.floor(x4)
+        c0, c1 = quartic((j - x4).astype(F32)), quartic(((j + F32(1)).astype(F32) - x4).astype(F32))
+        c0, c1 = np.where(np.isnan(c0), F32(0), c0), np.where(np.isnan(c1), F32(0), c1)  # max(NaN, 0) = 0
+        q = np.stack([e4m3(c0), e4m3((c1 - c0).astype(F32)), e4m3((F32(1) - c1).astype(F32)), np.zeros(len(x))], -1)
+        k = np.where(np.isnan(j), -2, np.clip(j, -2, 5)).astype(np.int64) + 2
+    byte = (np.array(tab, np.uint32)[k][:, None] >> (8 * np.arange(4, dtype=np.uint32))) & 0xFF
+    assert np.all((byte < 4) | (byte == 12))
+    return np.where(byte == 12, 0.0, np.take_along_axis(q, np.minimum(byte, 3).astype(np.int64), -1))
+
+
+def five_knot_fp8(x):
+    with np.errstate(all="ignore"):
+        x4 = (F32(4) * x).astype(F32)
+        c = [quartic((F32(k) - x4).astype(F32)) for k in range(5)]
+        c = [np.where(np.isnan(v), F32(0), v) for v in c]
+        return e4m3(np.stack([(c[b + 1] - c[b]).astype(F32) for b in range(4)], -1))
+
+
+def test_e4m3_quad_equals_the_five_knot_form():
+    """Every bin, the neighbourhoods of its edges (2^13 floats each way), the smallest and largest floats of
+    both signs, inputs out of range, infinities and NaNs.  (All 2^32 floats, in C: no difference.)"""
+    edges = np.array([-0.5, -0.25, 0.25, 0.5, 0.75, 1.0, 1.25, 1.5], F32).view(np.uint32).astype(np.int64)
+    near = (edges[:, None] + np.arange(-(1 << 13), (1 << 13) + 1)).ravel().astype(np.uint32).view(F32)
+    small = np.arange(0, 1 << 13, dtype=np.uint32).view(F32)
+    below = np.concatenate([-small, -np.exp2(np.random.default_rng(3).uniform(-40, -2, 200_000)).astype(F32)])
+    wide = np.random.default_rng(4).integers(0, 1 << 32, 400_000, dtype=np.uint64).astype(np.uint32).view(F32)
+    special = np.array([np.nan, -np.nan, np.inf, -np.inf, 3.4e38, -3.4e38, 0.0, -0.0, 1e-45], F32)
+    for x in (near, small, below, wide, special, np.random.default_rng(5).uniform(-0.6, 1.6, 400_000).astype(F32)):
+        a, b = five_knot_fp8(x), fp8_quad(x)
+        assert np.array_equal(a, b), x[(a != b).any(-1)][:5]
+    assert not five_knot_fp8(special[:4]).any()

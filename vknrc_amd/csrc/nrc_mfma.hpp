@@ -153,8 +153,12 @@ __device__ __forceinline__ uint32_t pack4_fp8(float a, float b, float c, float d
 }
 
 // The same quad as e4m3 bytes: one byte permute of (c_j, c_{j+1} - c_j, 1 - c_{j+1}, 0)
-// with the selectors of kOneBlobSel8.  The knots it leaves out change a feature by 6e-8 at
-// most (above), which is 0 in e4m3 (smallest value 2^-9).
+// with the selectors of kOneBlobSel8.  Over all 2^32 floats x it equals the five-knot form
+// rounded to e4m3: the knots are taken at j - 4x and (j + 1) - 4x, rounded as the five-knot
+// form rounds them (1 - f would round once more for x just below 0 and differ there for 23
+// floats), and a NaN gives the zero quad that clamping five NaN knots gives.  The knots that
+// are left out change a feature by 6e-8 at most (above), which is 0 in e4m3 (smallest value
+// 2^-9).
 constexpr uint32_t kOneBlobSel8[8] = {0x0C0C0C0Cu, 0x0C0C0C02u, 0x0C0C0201u, 0x0C020100u,
                                       0x0201000Cu, 0x01000C0Cu, 0x000C0C0Cu, 0x0C0C0C0Cu};
 
@@ -165,11 +169,11 @@ __device__ __forceinline__ void oneblob_sel8_init(uint32_t *tab, int lane) {
 __device__ __forceinline__ uint32_t oneblob4_fp8(float x, const uint32_t *sel) {
 	const float x4 = 4.0f * x;
 	const float j = __builtin_floorf(x4);
-	const float f = x4 - j;
-	const float c0 = quartic_cdf(-f), c1 = quartic_cdf(1.0f - f);
+	const float c0 = quartic_cdf(j - x4), c1 = quartic_cdf((j + 1.0f) - x4);
 	const uint32_t q = pack4_fp8(c0, c1 - c0, 1.0f - c1, 0.0f);
-	int k = (int)j; // saturating, NaN -> 0, as in oneblob4_packed
-	k = k < -2 ? -2 : (k > 5 ? 5 : k);
+	// clamped as a float: v_med3_f32 gives the smaller bound, and so the zero quad, for a NaN
+	// (the conversion to int would give 0, the quad of j = 0)
+	const int k = (int)__builtin_amdgcn_fmed3f(j, -2.0f, 5.0f);
 	return __builtin_amdgcn_perm(0u, q, sel[k + 2]);
 }
 
