@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "nrc_internal.hpp"
+#include "nrc_scratch.hpp"
 
 using nrc::DeviceState;
 
@@ -259,98 +260,10 @@ nrc_status check_train(nrc_cache *c, const nrc_train_record *d_records, uint32_t
 }
 
 
-// Scratch of the stateless gradient (nrc_mlp_gradient_f16): a few blocks per GPU kept
-// between calls, each guarded by the event of its last use.  A call takes a block that no
-// other host thread holds and that its own stream used last, or whose last use is over; it
-// makes its stream wait for that event and records the event again after its last kernel, so
-// calls on several streams and threads never share a block in use, nor wait for each other.
-// With no such block, or under stream capture, the scratch is stream-ordered as a library's
-// is (hipMallocAsync, hipFreeAsync).  Those two cost 25-40 us of host time a call: a forward
-// and a gradient of 16,384 rows took 109 us a pass with them, 33 us of it in kernels (38 us
-// a pass with a kept block).
-constexpr int kMaxDevices = 64, kScratchBlocks = 2;
-// one gradient workgroup a CU writes one row: 256 rows and both fragment copies, 21.3 MB
-constexpr size_t kScratchBytes = 2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDEN_LAYERS) + nrc::bwd_frag_halves(NRC_MAX_HIDDEN_LAYERS)) +
-                                 sizeof(float) * (((size_t)nrc::weight_count(NRC_MAX_HIDDEN_LAYERS) + 64) & ~size_t(63)) * 256;
-struct ScratchBlock {
-	void *p = nullptr;
-	hipEvent_t done = nullptr;
-	hipStream_t last = nullptr; // compared only: a reused handle still waits for `done`
-	bool held = false;
-};
-std::mutex g_scratch_mu;
-ScratchBlock g_scratch[kMaxDevices][kScratchBlocks];
-
-struct Scratch {
-	void *p = nullptr;
-	ScratchBlock *block = nullptr; // null: stream-ordered
-
-	static ScratchBlock *find(ScratchBlock (&blocks)[kScratchBlocks], hipStream_t s) {
-		for (ScratchBlock &b : blocks)
-			if (b.p && !b.held && b.last == s) return &b;
-		for (ScratchBlock &b : blocks) {
-			if (b.held) continue;
-			if (b.p) {
-				if (hipEventQuery(b.done) == hipSuccess) return &b;
-				continue;
-			}
-			if (hipEventCreateWithFlags(&b.done, hipEventDisableTiming) != hipSuccess) return nullptr;
-			if (hipMalloc(&b.p, kScratchBytes) == hipSuccess) return &b;
-			(void)hipEventDestroy(b.done);
-			b = ScratchBlock{};
-			return nullptr;
-		}
-		return nullptr;
-	}
-
-	hipError_t take(size_t bytes, hipStream_t s) {
-		int dev = 0;
-		hipError_t e = hipGetDevice(&dev);
-		if (e != hipSuccess) return e;
-		hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-		const bool captured = hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
-		if (!captured && bytes <= kScratchBytes && dev >= 0 && dev < kMaxDevices) {
-			std::lock_guard<std::mutex> lock(g_scratch_mu);
-			// relaxed: a capture that another stream has under way neither forbids nor sees
-			// the allocation and the queries
-			hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-			const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-			block = find(g_scratch[dev], s);
-			if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
-			if (block && hipStreamWaitEvent(s, block->done, 0) == hipSuccess) {
-				block->held = true;
-				p = block->p;
-				return hipSuccess;
-			}
-			block = nullptr;
-		}
-		(void)hipGetLastError();
-		return hipMallocAsync(&p, bytes, s);
-	}
-
-	// after the last kernel that uses the scratch was launched, whatever failed
-	hipError_t give(hipStream_t s) {
-		if (!block) return hipFreeAsync(p, s);
-		std::lock_guard<std::mutex> lock(g_scratch_mu);
-		const hipError_t e = hipEventRecord(block->done, s);
-		block->last = s;
-		if (e == hipSuccess) block->held = false; // a block whose use cannot be marked is never handed out again
-		return e;
-	}
-};
-
-// Frees the kept blocks of this GPU that no call holds (hipFree waits for their last use).
-void trim_scratch() {
-	int dev = 0;
-	if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return;
-	std::lock_guard<std::mutex> lock(g_scratch_mu);
-	for (ScratchBlock &b : g_scratch[dev])
-		if (b.p && !b.held) {
-			(void)hipFree(b.p);
-			(void)hipEventDestroy(b.done);
-			b = ScratchBlock{};
-		}
-}
+// Scratch of the stateless gradient (nrc_mlp_gradient_f16): one gradient workgroup a CU writes
+// one row, so a block holds 256 rows and both fragment copies, 21.3 MB
+nrc::ScratchPool g_scratch(2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDEN_LAYERS) + nrc::bwd_frag_halves(NRC_MAX_HIDDEN_LAYERS)) +
+                           sizeof(float) * (((size_t)nrc::weight_count(NRC_MAX_HIDDEN_LAYERS) + 64) & ~size_t(63)) * 256);
 
 // One training step on stream s (arguments already checked).
 nrc_status train_step(nrc_cache *c, const nrc_train_record *d_records, const uint32_t *d_count, uint32_t max_count,
@@ -492,7 +405,7 @@ nrc_status nrc_cache_create(const nrc_cache_desc *desc, nrc_cache **out) {
 		if (e != hipSuccess) return;
 		e = hipMalloc(p, bytes);
 		if (e != hipErrorOutOfMemory) return;
-		trim_scratch(); // kept scratch goes before a cache is refused
+		g_scratch.trim(); // kept scratch goes before a cache is refused
 		(void)hipGetLastError();
 		e = hipMalloc(p, bytes);
 	};
@@ -848,8 +761,8 @@ nrc_status nrc_mlp_gradient_f16(uint32_t hidden, const uint16_t *d_w, const uint
 	const uint32_t nb = nrc::plan_fused_gradient(n).blocks; // partial rows
 	const size_t nf = nrc::fwd_frag_halves((int)hidden), nt = nrc::bwd_frag_halves((int)hidden);
 	// the forward and the backward fragments and the partial rows
-	Scratch scr;
-	NRC_HIP(scr.take(2 * (nf + nt) + sizeof(float) * (size_t)pstride * nb, s), "gradient scratch");
+	nrc::ScratchPool::Lease scr;
+	NRC_HIP(g_scratch.take(scr, 2 * (nf + nt) + sizeof(float) * (size_t)pstride * nb, s), "gradient scratch");
 	_Float16 *wf = static_cast<_Float16 *>(scr.p), *wtf = wf + nf;
 	float *partials = reinterpret_cast<float *>(wtf + nt);
 	uint32_t nparts = 0;
@@ -858,7 +771,7 @@ nrc_status nrc_mlp_gradient_f16(uint32_t hidden, const uint16_t *d_w, const uint
 		e = nrc::launch_fused_gradient_f16((int)hidden, reinterpret_cast<const _Float16 *>(d_in), d_targets, n, wf, wtf,
 		                                   partials, pstride, &nparts, s);
 	if (e == hipSuccess) e = nrc::launch_reduce_partials(partials, nparts, pstride, wc, d_dw, s);
-	const hipError_t e2 = scr.give(s); // whatever failed
+	const hipError_t e2 = g_scratch.give(scr, s); // whatever failed
 	if (e != hipSuccess) return hip_fail(e, "nrc_mlp_gradient_f16");
 	if (e2 != hipSuccess) return hip_fail(e2, "nrc_mlp_gradient_f16 scratch");
 	return NRC_OK;
