@@ -415,6 +415,15 @@ nrc_status nrc_mlp_forward_f16(uint32_t hidden_layers, const uint16_t *d_weights
 nrc_status nrc_mlp_gradient_f16(uint32_t hidden_layers, const uint16_t *d_weights_f16, const uint16_t *d_inputs_f16,
                                 const float *d_targets, uint32_t n, float *d_dw, void *stream);
 
+/* No counterpart in the reference.  nrc_mlp_gradient_f16 keeps its device scratch
+ * between calls, at most two blocks of 21.3 MB a GPU (further calls in flight at the
+ * same time, calls under stream capture and calls on a stream of another GPU than the
+ * current one take stream-ordered memory).  This frees the blocks of the current GPU,
+ * waiting for the kernels that use them; a block that a call on another host thread
+ * holds stays.  The library frees them by itself before one of its own allocations is
+ * refused. */
+nrc_status nrc_release_scratch(void);
+
 /* Largest n nrc_mlp_gradient_f16_noalloc takes (its scratch is sized for it). */
 #define NRC_NOALLOC_MAX_GRADIENT_RECORDS 16384u
 

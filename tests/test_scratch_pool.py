@@ -124,3 +124,34 @@ def test_scratch_of_the_default_streams(tmp_path, handle):
 	CHECK(pool.give(b, {handle}) == hipSuccess && pool.give(big, {handle}) == hipSuccess);
 	CHECK(g_last == hipSuccess && g_live.size() == 1);
 	return 0;""")
+
+
+# idle blocks go before an allocation of the library or a stream-ordered one is refused, and when they are
+# asked for; a block in a call's hands stays, and so does an error that trimming cannot help
+def test_scratch_is_given_back(tmp_path):
+    run(tmp_path, """
+	g_free[0] = 250;
+	ihipStream_t s{0, false}, t{0, false};
+	nrc::ScratchPool::Lease a, b, big;
+	CHECK(pool.take(a, 50, &s) == hipSuccess && pool.take(b, 50, &t) == hipSuccess && g_free[0] == 50);
+	CHECK(pool.give(a, &s) == hipSuccess);
+	void *p = nullptr, *q = nullptr;
+	CHECK(pool.malloc(&p, 120) == hipSuccess && g_free[0] == 30); // a's block went, b's is held
+	CHECK(pool.malloc(&q, 120) == hipErrorOutOfMemory);
+	CHECK(pool.give(b, &t) == hipSuccess && pool.malloc(&q, 120) == hipSuccess && g_free[0] == 10);
+	CHECK(hipFree(p) == hipSuccess && hipFree(q) == hipSuccess && g_live.empty());
+
+	g_last = hipSuccess;
+	CHECK(pool.take(a, 50, &s) == hipSuccess && pool.give(a, &s) == hipSuccess && g_free[0] == 150);
+	CHECK(pool.take(big, 240, &s) == hipSuccess && g_live.at(big.p).ordered && g_free[0] == 10);
+	CHECK(g_last == hipSuccess && pool.give(big, &s) == hipSuccess);
+	CHECK(pool.take(a, 50, &s) == hipSuccess && pool.give(a, &s) == hipSuccess);
+	pool.trim();
+	CHECK(g_live.empty() && g_free[0] == 250);
+	return 0;""")
+
+
+# the library's own allocations all go through the pool, so none is refused while idle scratch is kept
+def test_library_allocations_go_through_the_pool():
+    src = open(os.path.join(ROOT, "vknrc_amd", "csrc", "nrc_api.cpp")).read()
+    assert "g_scratch.malloc(" in src and "hipMalloc(" not in src and "hipExtMalloc" not in src

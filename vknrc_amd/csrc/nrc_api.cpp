@@ -175,24 +175,29 @@ nrc::AdamParams adam_params(const nrc_cache *c) {
 	return p;
 }
 
+// Scratch of the stateless gradient (nrc_mlp_gradient_f16): one gradient workgroup a CU writes
+// one row, so a block holds 256 rows and both fragment copies, 21.3 MB
+nrc::ScratchPool g_scratch(2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDEN_LAYERS) + nrc::bwd_frag_halves(NRC_MAX_HIDDEN_LAYERS)) +
+                           sizeof(float) * (((size_t)nrc::weight_count(NRC_MAX_HIDDEN_LAYERS) + 64) & ~size_t(63)) * 256);
+
 // The plain path's scratch, allocated on its first use.  All three buffers are set
 // together or not at all, so a failed attempt leaves the cache as it was.
 nrc_status ensure_plain_scratch(nrc_cache *c) {
 	if (c->acts) return NRC_OK;
 	const uint32_t ldn = (c->desc.train_batch_size + 63u) & ~63u;
 	const size_t slab = (size_t)(c->desc.hidden_layers + 1) * 64 * ldn;
-	float *acts = nullptr, *deltas = nullptr, *loss = nullptr;
-	hipError_t e = hipMalloc(&acts, slab * sizeof(float));
-	if (e == hipSuccess) e = hipMalloc(&deltas, slab * sizeof(float));
-	if (e == hipSuccess) e = hipMalloc(&loss, (size_t)ldn * sizeof(float));
+	void *acts = nullptr, *deltas = nullptr, *loss = nullptr;
+	hipError_t e = g_scratch.malloc(&acts, slab * sizeof(float));
+	if (e == hipSuccess) e = g_scratch.malloc(&deltas, slab * sizeof(float));
+	if (e == hipSuccess) e = g_scratch.malloc(&loss, (size_t)ldn * sizeof(float));
 	if (e != hipSuccess) {
-		for (float *p : {acts, deltas, loss})
+		for (void *p : {acts, deltas, loss})
 			if (p) (void)hipFree(p);
 		return hip_fail(e, "plain scratch");
 	}
-	c->acts = acts;
-	c->deltas = deltas;
-	c->sample_loss = loss;
+	c->acts = static_cast<float *>(acts);
+	c->deltas = static_cast<float *>(deltas);
+	c->sample_loss = static_cast<float *>(loss);
 	c->ldn = ldn;
 	return NRC_OK;
 }
@@ -259,11 +264,6 @@ nrc_status check_train(nrc_cache *c, const nrc_train_record *d_records, uint32_t
 	return NRC_OK;
 }
 
-
-// Scratch of the stateless gradient (nrc_mlp_gradient_f16): one gradient workgroup a CU writes
-// one row, so a block holds 256 rows and both fragment copies, 21.3 MB
-nrc::ScratchPool g_scratch(2 * (size_t)(nrc::fwd_frag_halves(NRC_MAX_HIDDEN_LAYERS) + nrc::bwd_frag_halves(NRC_MAX_HIDDEN_LAYERS)) +
-                           sizeof(float) * (((size_t)nrc::weight_count(NRC_MAX_HIDDEN_LAYERS) + 64) & ~size_t(63)) * 256);
 
 // One training step on stream s (arguments already checked).
 nrc_status train_step(nrc_cache *c, const nrc_train_record *d_records, const uint32_t *d_count, uint32_t max_count,
@@ -402,12 +402,7 @@ nrc_status nrc_cache_create(const nrc_cache_desc *desc, nrc_cache **out) {
 	const CacheSizes sz(*desc);
 	hipError_t e = hipGetDevice(&c->device);
 	auto alloc = [&](auto **p, size_t bytes) {
-		if (e != hipSuccess) return;
-		e = hipMalloc(p, bytes);
-		if (e != hipErrorOutOfMemory) return;
-		g_scratch.trim(); // kept scratch goes before a cache is refused
-		(void)hipGetLastError();
-		e = hipMalloc(p, bytes);
+		if (e == hipSuccess) e = g_scratch.malloc(reinterpret_cast<void **>(p), bytes);
 	};
 	alloc(&c->entries, sz.entries);
 	alloc(&c->w16, sz.w16);
@@ -774,6 +769,11 @@ nrc_status nrc_mlp_gradient_f16(uint32_t hidden, const uint16_t *d_w, const uint
 	const hipError_t e2 = g_scratch.give(scr, s); // whatever failed
 	if (e != hipSuccess) return hip_fail(e, "nrc_mlp_gradient_f16");
 	if (e2 != hipSuccess) return hip_fail(e2, "nrc_mlp_gradient_f16 scratch");
+	return NRC_OK;
+}
+
+nrc_status nrc_release_scratch(void) {
+	g_scratch.trim();
 	return NRC_OK;
 }
 

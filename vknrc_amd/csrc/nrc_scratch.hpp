@@ -65,7 +65,13 @@ public:
 			}
 		}
 		(void)hipGetLastError();
-		return hipMallocAsync(&l.p, bytes, s);
+		hipError_t m = hipMallocAsync(&l.p, bytes, s);
+		if (m == hipErrorOutOfMemory && !captured) {
+			trim();
+			(void)hipGetLastError();
+			m = hipMallocAsync(&l.p, bytes, s);
+		}
+		return m;
 	}
 
 	// after the last kernel that uses the scratch was launched, whatever failed
@@ -79,17 +85,30 @@ public:
 		return e;
 	}
 
-	// Frees the kept blocks of this GPU that no call holds (hipFree waits for their last use).
+	// Frees the kept blocks of this GPU that no call holds (hipFree waits for their last use);
+	// a capture that is under way elsewhere is not disturbed.
 	void trim() {
 		int dev = 0;
 		if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return;
 		std::lock_guard<std::mutex> lock(mu_);
+		hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+		const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
 		for (Block &b : blocks_[dev])
 			if (b.p && !b.held) {
 				(void)hipFree(b.p);
 				(void)hipEventDestroy(b.done);
 				b = Block{};
 			}
+		if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+	}
+
+	// hipMalloc for the library's other allocations: the kept blocks go before one is refused
+	hipError_t malloc(void **p, size_t bytes) {
+		hipError_t e = hipMalloc(p, bytes);
+		if (e != hipErrorOutOfMemory) return e;
+		trim();
+		(void)hipGetLastError();
+		return hipMalloc(p, bytes);
 	}
 
 private:

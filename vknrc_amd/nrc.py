@@ -158,6 +158,7 @@ def load_library():
     L.nrc_screen_tonemap.argtypes = [P, P, U32, U32, U32, I32, U32, P, P]
     L.nrc_mlp_gradient_f16.argtypes = [U32, P, P, P, U32, P, P]
     L.nrc_mlp_gradient_f16_noalloc.argtypes = [U32, P, P, P, U32, P, P]
+    L.nrc_release_scratch.argtypes = []
     GI = C.POINTER(GroupItem)
     L.nrc_group_infer.argtypes = [GI, U32, C.c_int, P]
     L.nrc_group_train.argtypes = [GI, U32, U32, C.c_int, U32, P]
@@ -169,6 +170,7 @@ def load_library():
     for f in ("nrc_init_weights", "nrc_cache_create", "nrc_cache_reset", "nrc_cache_get_desc", "nrc_set_use_ema",
               "nrc_infer", "nrc_train", "nrc_frame", "nrc_get_state", "nrc_set_state", "nrc_encode",
               "nrc_sph_encode", "nrc_mlp_forward_f16", "nrc_mlp_gradient_f16", "nrc_mlp_gradient_f16_noalloc",
+              "nrc_release_scratch",
               "nrc_group_infer", "nrc_scene_pack_primitives", "nrc_unpack_eval_records", "nrc_unpack_train_records",
               "nrc_composite_records",
               "nrc_build_train_records", "nrc_screen_tonemap",
@@ -529,6 +531,11 @@ def mlp_forward_f16(weights_f16, inputs_f16, n: int, out, hidden_layers: int = 5
 def mlp_gradient_f16(weights_f16, inputs_f16, targets, n: int, dw, hidden_layers: int = 5, stream=None) -> None:
     _check(load_library().nrc_mlp_gradient_f16(int(hidden_layers), _ptr(weights_f16), _ptr(inputs_f16),
                                                _ptr(targets), int(n), _ptr(dw), _stream(stream)))
+
+
+def release_scratch() -> None:
+    """Frees the device scratch that mlp_gradient_f16 keeps on the current GPU (nrc_release_scratch)."""
+    _check(load_library().nrc_release_scratch())
 
 
 def mlp_gradient_f16_noalloc(weights_f16, inputs_f16, targets, n: int, dw, hidden_layers: int = 5,
