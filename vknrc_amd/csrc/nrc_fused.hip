@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "nrc_grad_rows.hpp"
 #include "nrc_mfma.hpp"
 
 #include <atomic>
@@ -1314,22 +1315,18 @@ template <int H, int ENC, int LOSS, bool F16IN> hipError_t grad_small_attributes
 template <int H, int ENC, int LOSS, bool F16IN> hipError_t grad_small_launch(GradGroup &grp, hipStream_t s) {
 	const size_t smem = sizeof(SmallGradSmem<H>);
 	bool multi = false;
-	uint32_t rows = 0, pairs = 0;
+	GradRows rows[kGroupMax];
 	for (uint32_t i = 0; i < grp.n_items; ++i) {
-		multi |= grp.item[i].chunks > 1;
-		rows += grp.item[i].blocks;
-		pairs += (grp.item[i].blocks + 1) / 2;
+		const GradItem &it = grp.item[i];
+		const uint32_t n = it.max_count < it.clamp ? it.max_count : it.clamp;
+		const uint32_t chunks = n == 0 ? 1u : (n + kFusedSmallRecords - 1) / kFusedSmallRecords;
+		multi |= it.chunks > 1;
+		rows[i] = GradRows{it.blocks, it.chunks < chunks ? it.chunks : chunks};
 	}
-	// One row a CU (fused_grad_small_kernel), or two rows side by side (the same bits).  Rows
-	// run in rounds of one workgroup a CU, and a round of pairs takes 1.57 times a round of
-	// single rows (8 chunks a row: 67 us against 42.6), so the pairs win where they save more
-	// than that in rounds: 272 and 293 rows of 8 chunks 1.13x a 16-cache frame, 288 of 2 chunks
-	// 1.12x; not up to one row a CU, nor where both need a nearly empty last round (528 and 640
-	// rows: three rounds against two).  Rows of one chunk stay single: 512 to 1,984 of them
-	// took 0.95x a frame in pairs, which store all their sums at the end of a short row where
-	// the one-chunk kernel's stores drain during its backward.
-	const uint32_t cus = (uint32_t)device_cu_count();
-	const bool dual = !F16IN && multi && 8 * ((pairs + cus - 1) / cus) < 5 * ((rows + cus - 1) / cus);
+	// A launch of one-chunk rows alone keeps the one-chunk kernel, whose stores drain during its
+	// backward: 512 to 1,984 such rows took 0.95x a frame in pairs, which store all their sums at
+	// the end.
+	const bool dual = !F16IN && multi && grad_rows_in_pairs<kGroupMax>(rows, grp.n_items, (uint32_t)device_cu_count());
 	grp.total_blocks = 0;
 	for (uint32_t i = 0; i < grp.n_items; ++i) {
 		grp.item[i].block_begin = grp.total_blocks;
