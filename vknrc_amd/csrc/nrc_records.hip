@@ -145,6 +145,16 @@ __device__ __forceinline__ void transform_vertex(const float *T, const float *v,
 	for (int j = 0; j < 3; ++j) o[j] = T[4 * j] * v[0] + T[4 * j + 1] * v[1] + T[4 * j + 2] * v[2] + T[4 * j + 3];
 }
 
+// Opaque values, so that the compiler fuses the products of a packed record into the sums as
+// it does those of the index arrays: either way gives the same bits
+__device__ __forceinline__ void opaque(PrimitiveData &d) {
+#pragma unroll
+	for (int k = 0; k < 3; ++k) {
+		asm volatile("" : "+v"(d.c[k][0]), "+v"(d.c[k][1]), "+v"(d.c[k][2]));
+		asm volatile("" : "+v"(d.t[k][0]), "+v"(d.t[k][1]));
+	}
+}
+
 // UnpackNRCInput (NRCRecord.glsl:98-125) into the 14 floats of an nrc_query
 template <bool PACKED>
 __device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, const float *lut, float *q) {
@@ -156,52 +166,69 @@ __device__ void unpack_input(const nrc_scene &s, const nrc_packed_input &p, cons
 	PrimitiveData d;
 	if constexpr (PACKED) d = packed_primitive(s.d_primitives + prim);
 	else d = indexed_primitive(s, prim);
-	// opaque values, so that the compiler fuses the products below into the sums in the same
-	// way whichever way they were loaded: the packed records give the bits of the index arrays
-#pragma unroll
-	for (int k = 0; k < 3; ++k) {
-		asm volatile("" : "+v"(d.c[k][0]), "+v"(d.c[k][1]), "+v"(d.c[k][2]));
-		asm volatile("" : "+v"(d.t[k][0]), "+v"(d.t[k][1]));
-	}
-	const nrc_material *m = s.d_materials + d.material;
-	const f4v mat[2] = {record_piece(m, 0), record_piece(m, 1)};
-	const float roughness = m->roughness;
-	const float diffuse[3] = {mat[0][0], mat[0][1], mat[0][2]}, specular[3] = {mat[1][0], mat[1][1], mat[1][2]};
-	const float dt = mat[0][3], st = mat[1][3];
-	const uint32_t tex[2] = {__float_as_uint(dt), __float_as_uint(st)};
-	nrc_texture t[2] = {};
-	bool valid[2];
-#pragma unroll
-	for (int k = 0; k < 2; ++k) {
-		valid[k] = texture_id_valid(s, tex[k]);
-		if (valid[k]) t[k] = s.d_textures[tex[k]];
-	}
 	float b[3];
 	unorm2x16(p.barycentric_2x16u, b + 1);
 	b[0] = 1.0f - b[1] - b[2];
-	const float u = d.t[0][0] * b[0] + d.t[1][0] * b[1] + d.t[2][0] * b[2];
-	const float v = d.t[0][1] * b[0] + d.t[1][1] * b[1] + d.t[2][1] * b[2];
+	// the material's two textures, their texels under way
+	float roughness, diffuse[3], specular[3];
 	TexelFetch texels[2];
+	auto surface = [&]() __attribute__((always_inline)) {
+		const nrc_material *m = s.d_materials + d.material;
+		const f4v mat[2] = {record_piece(m, 0), record_piece(m, 1)};
+		roughness = m->roughness;
 #pragma unroll
-	for (int k = 0; k < 2; ++k) texels[k].fetch(t[k], valid[k], u, v);
-	const float T[12] = {rows[0][0], rows[0][1], rows[0][2], rows[0][3], rows[1][0], rows[1][1],
-	                     rows[1][2], rows[1][3], rows[2][0], rows[2][1], rows[2][2], rows[2][3]};
-	float v0[3], v1[3], v2[3];
-	transform_vertex(T, d.c[0], v0);
-	transform_vertex(T, d.c[1], v1);
-	transform_vertex(T, d.c[2], v2);
-	const float e1[3] = {v1[0] - v0[0], v1[1] - v0[1], v1[2] - v0[2]};
-	const float e2[3] = {v2[0] - v0[0], v2[1] - v0[1], v2[2] - v0[2]};
-	float n[3] = {e1[1] * e2[2] - e1[2] * e2[1], e1[2] * e2[0] - e1[0] * e2[2], e1[0] * e2[1] - e1[1] * e2[0]};
-	const float inv = 1.0f / sqrtf(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-	const float sgn = flip ? -inv : inv;
-	n[0] *= sgn;
-	n[1] *= sgn;
-	n[2] *= sgn;
+		for (int j = 0; j < 3; ++j) {
+			diffuse[j] = mat[0][j];
+			specular[j] = mat[1][j];
+		}
+		const float dt = mat[0][3], st = mat[1][3];
+		const uint32_t tex[2] = {__float_as_uint(dt), __float_as_uint(st)};
+		nrc_texture t[2] = {};
+		bool valid[2];
 #pragma unroll
-	for (int j = 0; j < 3; ++j) q[j] = v0[j] * b[0] + v1[j] * b[1] + v2[j] * b[2];
-	unorm2x16(p.scattered_dir_2x16u, q + 3);
-	sph_encode(n[0], n[1], n[2], q + 5);
+		for (int k = 0; k < 2; ++k) {
+			valid[k] = texture_id_valid(s, tex[k]);
+			if (valid[k]) t[k] = s.d_textures[tex[k]];
+		}
+		const float u = d.t[0][0] * b[0] + d.t[1][0] * b[1] + d.t[2][0] * b[2];
+		const float v = d.t[0][1] * b[0] + d.t[1][1] * b[1] + d.t[2][1] * b[2];
+#pragma unroll
+		for (int k = 0; k < 2; ++k) texels[k].fetch(t[k], valid[k], u, v);
+	};
+	// world position and the angles of the normal
+	auto geometry = [&]() __attribute__((always_inline)) {
+		const float T[12] = {rows[0][0], rows[0][1], rows[0][2], rows[0][3], rows[1][0], rows[1][1],
+		                     rows[1][2], rows[1][3], rows[2][0], rows[2][1], rows[2][2], rows[2][3]};
+		float v0[3], v1[3], v2[3];
+		transform_vertex(T, d.c[0], v0);
+		transform_vertex(T, d.c[1], v1);
+		transform_vertex(T, d.c[2], v2);
+		const float e1[3] = {v1[0] - v0[0], v1[1] - v0[1], v1[2] - v0[2]};
+		const float e2[3] = {v2[0] - v0[0], v2[1] - v0[1], v2[2] - v0[2]};
+		float n[3] = {e1[1] * e2[2] - e1[2] * e2[1], e1[2] * e2[0] - e1[0] * e2[2], e1[0] * e2[1] - e1[1] * e2[0]};
+		const float inv = 1.0f / sqrtf(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+		const float sgn = flip ? -inv : inv;
+		n[0] *= sgn;
+		n[1] *= sgn;
+		n[2] *= sgn;
+#pragma unroll
+		for (int j = 0; j < 3; ++j) q[j] = v0[j] * b[0] + v1[j] * b[1] + v2[j] * b[2];
+		unorm2x16(p.scattered_dir_2x16u, q + 3);
+		sph_encode(n[0], n[1], n[2], q + 5);
+	};
+	// A packed record arrives whole, and the chain material, texture, texels has the geometry to
+	// hide behind.  Through the index arrays six gathers arrive one by one: the corners' work
+	// starts before the texture coordinates are there, in 13 registers less (2,073,600 eval
+	// records of 4,096 primitives 94.4 -> 80.2 us, of a million 325 -> 308; with the material
+	// first 96.5 and 325).
+	if constexpr (PACKED) {
+		opaque(d);
+		surface();
+		geometry();
+	} else {
+		geometry();
+		surface();
+	}
 	q[7] = roughness;
 	texels[0].color(diffuse, lut, q + 8);
 	texels[1].color(specular, lut, q + 11);
@@ -227,9 +254,9 @@ __device__ __forceinline__ nrc_packed_input load_packed(const uint32_t *w) {
 // look-ups, the vector unit (690 instructions a record) and the misses of L2 (1.3 a record),
 // each busy for over half of the time; the chain record, primitive, material, texture, texels
 // has the next record's loads to hide behind in a large launch only, so what does not depend
-// on each other is loaded together (both textures before the geometry is worked out).
-// Random packed primitives: 2,073,600 eval records 80 -> 64 us, 65,536 train records
-// 7.0 -> 5.8 us; indexed primitives 151 -> 141 and 9.6 -> 9.2 us.
+// on each other is loaded together (both textures, and of packed primitives before the geometry
+// is worked out).  65,536 random primitives: 2,073,600 eval records 81 -> 64 us packed and
+// 159 -> 142 indexed, 65,536 train records 7.2 -> 6.2 and 9.6 -> 8.7.
 constexpr uint32_t kUnpackWaves = 4;
 template <bool PACKED, bool STAGED, int WORDS, int AT, int FLOATS>
 __global__ __launch_bounds__(64 * kUnpackWaves) void unpack_kernel(const nrc_scene s, const uint32_t *__restrict__ rec,
@@ -447,9 +474,10 @@ hipError_t launch_unpack(const nrc_scene &s, const void *rec, const uint32_t *d_
 	const dim3 grid((max_count + 64u * kUnpackWaves - 1u) / (64u * kUnpackWaves)), block(64 * kUnpackWaves);
 	const uint32_t *r = static_cast<const uint32_t *>(rec);
 	// Up to half a wave a SIMD (32,768 records) nothing hides the two passes through LDS, and the
-	// vector cache has look-ups to spare.  Straight and staged: 4,096 train records 5.14 and
-	// 5.64 us on packed primitives, 5.9 and 6.4 on indexed ones; 16,384 eval records 5.25 and
-	// 5.31, 6.0 and 6.5; 65,536 train records 6.37 and 6.30; 230,400 eval records 12.4 and 11.4.
+	// vector cache has look-ups to spare.  Straight and staged: 4,096 train records 5.0 and
+	// 5.3 us on packed primitives, 5.8 and 6.2 on indexed ones; 16,384 eval records 4.8 and
+	// 5.3, 5.8 and 6.2; 65,536 train records 6.6 and 6.3, 8.8 and 8.7; 230,400 eval records
+	// 12.8 and 11.9, 21.0 and 20.9.
 	const bool staged = (uint64_t)grid.x * kUnpackWaves > 2u * (uint64_t)device_cu_count();
 	if (s.d_primitives)
 		staged ? unpack_kernel<true, true, WORDS, AT, FLOATS><<<grid, block, 0, stream>>>(s, r, d_count, max_count, out)
