@@ -386,6 +386,7 @@ template <int H, int ENC> hipError_t fp8_launch(InferGroup &grp, const Fp8PrepGr
 	if (cap > (uint32_t)kFp8MaxBlocks) cap = kFp8MaxBlocks;
 	if (blocks > cap) blocks = cap;
 	if (blocks == 0) blocks = 1;
+	grp.deal = deals_by_count(grp, blocks) ? kDealByCount : kDealByMaximum;
 	fp8_infer_kernel<H, ENC><<<dim3(blocks), dim3(256), 0, s>>>(grp);
 	return hipGetLastError();
 }

@@ -1275,12 +1275,13 @@ bool infer_pipelined() {
 	return p;
 }
 
-template <int H, int ENC, bool F16IN> hipError_t infer_launch(const InferGroup &grp, hipStream_t s) {
+template <int H, int ENC, bool F16IN> hipError_t infer_launch(InferGroup &grp, hipStream_t s) {
 	// persistent: a few workgroups per CU, each wave a contiguous tile range
 	uint32_t blocks = (grp.total_tiles + 3) / 4;
 	const uint32_t cap = (uint32_t)device_cu_count() * infer_wg_per_cu();
 	if (blocks > cap) blocks = cap;
 	if (blocks == 0) blocks = 1;
+	grp.deal = deals_by_count(grp, blocks) ? infer_deal_limits(grp.total_tiles, 4 * blocks, infer_wg_per_cu()) : kDealByMaximum;
 	if (!F16IN && infer_pipelined())
 		fused_infer_pipe_kernel<H, ENC><<<dim3(blocks), dim3(256), 0, s>>>(grp);
 	else if (infer_tiles_override() == 1)
@@ -1365,7 +1366,7 @@ template <int H> hipError_t grad_group_h(int encoding, int loss, GradGroup &g, h
 	}
 }
 
-template <int H> hipError_t infer_h(int enc, const InferGroup &grp, hipStream_t s) {
+template <int H> hipError_t infer_h(int enc, InferGroup &grp, hipStream_t s) {
 	switch (enc) {
 	case NRC_ENCODING_TRI12: return infer_launch<H, NRC_ENCODING_TRI12, false>(grp, s);
 	case NRC_ENCODING_SINCOS6: return infer_launch<H, NRC_ENCODING_SINCOS6, false>(grp, s);

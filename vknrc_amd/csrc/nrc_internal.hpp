@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "nrc.h"
+#include "nrc_deal.hpp"
 #include "nrc_device.hpp"
 
 namespace nrc {
@@ -60,8 +61,16 @@ struct InferGroup {
 	InferItem item[kGroupMax];
 	const _Float16 *fin; // pre-encoded fp16 inputs [n][64] (single-item test entry point only)
 	uint32_t n_items, total_tiles;
-	int clamp0; // max(pred, 0) as nrc_inference.comp:48
+	DealLimits deal; // which device counts are dealt instead of the maximum
+	int clamp0;      // max(pred, 0) as nrc_inference.comp:48
 };
+
+// Whether an inference on `blocks` workgroups of 4 waves may deal its tiles by a device count: one
+// cache with a count, and more tiles than waves (else a wave has one at most either way).  The
+// counts of several caches would have to be fetched one after the other first.
+inline bool deals_by_count(const InferGroup &grp, uint32_t blocks) {
+	return grp.n_items == 1 && grp.item[0].d_count != nullptr && grp.total_tiles > 4 * blocks;
+}
 
 // One cache's share of a grouped fused gradient.
 struct GradItem {

@@ -51,16 +51,21 @@ __device__ __forceinline__ half8_t pack_relu(float4_t lo, float4_t hi) {
 }
 
 // The tiles that an inference launch deals to its waves.  One cache with more tiles than
-// waves: those of the records that there are (the device count), so that a count below the
-// maximum leaves no wave without work (700,001 of 921,600 queries: 36.1 us dealt by the
-// maximum, 33.0 by the count).  No more tiles than waves: a wave has one at most either way,
-// and the count would only be one more load to wait for first (1,000 queries: the kernel
-// takes 6.36 us, 6.44 with it).  Several caches: the maxima's, which the host has added up;
-// the counts of all of them would have to be fetched one after the other first.
+// waves: those of the records that there are (the device count) where grp.deal says so
+// (nrc_deal.hpp), else those of the maximum.  No more tiles than waves: a wave has one at
+// most either way, and the count would only be one more load to wait for first (1,000
+// queries: the kernel takes 6.36 us, 6.44 with it).  Several caches: the maxima's, which the
+// host has added up; the counts of all of them would have to be fetched one after the other
+// first.
 __device__ __forceinline__ uint32_t infer_tiles(const InferGroup &grp) {
-	if (grp.n_items != 1 || grp.total_tiles <= gridDim.x * 4u) return grp.total_tiles;
-	const InferItem &it = grp.item[0];
-	return (__builtin_amdgcn_readfirstlane(effective_count(it.d_count, it.max_count, it.max_count)) + 63u) / 64u;
+	const uint32_t *d_count = grp.item[0].d_count;
+	const uint32_t total = grp.total_tiles, max_count = grp.item[0].max_count;
+	const uint32_t split = grp.deal.split, all = grp.deal.all, some = grp.deal.some;
+	// every argument at once, ahead of the branches that would fetch them one after the other
+	asm volatile("" ::"s"(d_count), "s"(total), "s"(max_count), "s"(split), "s"(all), "s"(some));
+	if (all == 0u) return total; // uniform
+	const uint32_t tiles = (__builtin_amdgcn_readfirstlane(effective_count(d_count, max_count, max_count)) + 63u) / 64u;
+	return tiles <= (tiles > split ? all : some) ? tiles : total;
 }
 
 // Calls f(std::integral_constant<int, i>{}) for i = 0 .. N-1, unrolled at compile time.
