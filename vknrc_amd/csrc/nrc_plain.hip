@@ -201,7 +201,8 @@ __global__ __launch_bounds__(64 * kPlainInferWaves) void plain_infer_kernel(cons
 		const uint32_t n = tile < tiles ? tile * 16 + r : last;
 		load_query(queries + (size_t)(n < last ? n : last) * kQueryFloats, rec);
 	};
-	if (count > 0) load_tile(t); // uniform
+	if (blockIdx.x >= tiles) return; // no tile for any wave: nothing to stage the weights for (uniform)
+	load_tile(t);
 	stage_weights<H, kPlainInferWaves>(S, w32);
 	float4_t next[4];
 	layer_fragments<H>(S, 0, 0, slot, next);
@@ -263,7 +264,8 @@ __global__ __launch_bounds__(64 * kPlainWaves) void plain_fwdbwd_kernel(const fl
 #pragma unroll
 		for (int i = 0; i < kTrainFloats; ++i) rec[i] = rp[i];
 	};
-	if (count > 0) load_tile(t); // uniform; on their way while the weights are staged
+	if (blockIdx.x >= tiles) return; // no tile for any wave: nothing to stage the weights for (uniform)
+	load_tile(t); // on their way while the weights are staged
 	stage_weights<H, kPlainWaves>(S, w32);
 	float4_t next[4];
 	layer_fragments<H>(S, 0, 0, slot, next);
