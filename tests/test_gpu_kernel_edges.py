@@ -84,8 +84,8 @@ def test_mlp_gradient_streams():
     assert np.array_equal(host(many), host(one))
 
 
-# the forward gathers row-major weights with wide loads where their address allows it and
-# single halves where it does not: the same fragments, so the same bits
+# the forward reads row-major weights with 16-byte loads at any alignment and puts them into LDS
+# in fragment order: the same fragments, so the same bits
 @pytest.mark.parametrize("hidden", [4, 5])
 @pytest.mark.parametrize("n", [1, 63, 65, 4097])
 def test_mlp_forward_weight_alignment(hidden, n):
@@ -137,8 +137,9 @@ def test_plain_inference_tiles(hidden, enc, n, live):
     st.close()
 
 
-# the chunks of the FP32 weight gradient: inside one tile, at its edges, at the edges of a
-# 256-record chunk, many chunks with a partial last one, and a device count below the size
+# the FP32 weight gradient: inside one tile, at its edges, half a 512-record chunk and one record more,
+# many chunks with a partial last one, and a device count below the size (the edges of a chunk are
+# test_gpu_later_tiles.py's)
 @pytest.mark.parametrize("hidden,enc", ENCODINGS)
 @pytest.mark.parametrize("n,live", [(1, 1), (16, 16), (17, 17), (256, 256), (257, 257), (8193, 8100)])
 def test_plain_gradient_chunks(hidden, enc, n, live):
@@ -225,9 +226,10 @@ def test_unpack_partial_waves(packed, room):
         assert np.array_equal(rows(v.unpack_train_records, tr, 17, n, live), trained[:live]), n
 
 
-# more multi-chunk rows than CUs run two a workgroup: caches with an odd number of rows, a single
-# row, a partial last chunk, device counts that leave a row's last chunk or whole rows empty, and a
-# chunk whose deltas carry a scale, each with the bits that the cache has alone
+# a group of multi-chunk rows in three rounds, which run one a workgroup on 256 CUs (two a workgroup:
+# test_gpu_row_pairs.py): caches with an odd number of rows, a single row, a partial last chunk, device
+# counts that leave a row's last chunk or whole rows empty, and a chunk whose deltas carry a scale, each with
+# the bits that the cache has alone
 @pytest.mark.parametrize("hidden,enc", ENCODINGS)
 @pytest.mark.parametrize("loss", [v.LOSS_RELATIVE_L2_LUMINANCE, v.LOSS_L2])
 def test_gradient_row_pairs(hidden, enc, loss):

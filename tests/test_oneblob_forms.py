@@ -1,5 +1,5 @@
 """Pins the inference kernels' two-knot one-blob encoder (oneblob4_packed, nrc_mfma.hpp) against the
-five-knot form of NRCOneBlob4Encode (shader/src/NRCRecord.glsl:51-63, the form of oneblob4_knots), both
+five-knot form of NRCOneBlob4Encode (shader/src/NRCRecord.glsl:51-63), both
 restated here in FP32 with fused multiply-adds as the kernels compute them, and the byte-permute selector
 table kOneBlobSel (read from the header) against the placement it must produce.
 
@@ -42,7 +42,7 @@ def quartic(u):
 
 
 def five_knot(x):
-    """oneblob4_knots: the knots k - 4x, k = 0..4 (4x is exact, one rounding), differences in FP32."""
+    """The knots k - 4x, k = 0..4 (4x is exact, one rounding), differences in FP32."""
     x4 = (F32(4) * x).astype(F32)
     c = [quartic((F32(k) - x4).astype(F32)) for k in range(5)]
     return np.stack([(c[b + 1] - c[b]).astype(F32) for b in range(4)], -1)

@@ -386,6 +386,10 @@ template <int H, int ENC> hipError_t fp8_launch(InferGroup &grp, const Fp8PrepGr
 	if (cap > (uint32_t)kFp8MaxBlocks) cap = kFp8MaxBlocks;
 	if (blocks > cap) blocks = cap;
 	if (blocks == 0) blocks = 1;
+	// Every count: a workgroup copies the weights to LDS once whatever it runs, so an even deal
+	// costs little and saves most (of 131 sizes and counts 0.88 of the time of the maximum's deal
+	// in the mean: 524,288 queries of which 131,072, 15.4 -> 10.7 us; 196,608 of 393,216, 14.0 -> 15.1,
+	// is the worst).
 	grp.deal = deals_by_count(grp, blocks) ? kDealByCount : kDealByMaximum;
 	fp8_infer_kernel<H, ENC><<<dim3(blocks), dim3(256), 0, s>>>(grp);
 	return hipGetLastError();

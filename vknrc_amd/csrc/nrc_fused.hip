@@ -917,9 +917,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // each split in its two 4-half runs (256 halves of a block, then 256): the forward reads both
 // runs, 512 contiguous bytes each, and the backward's W_l^T fragments come from transposing
 // reads of one run, which also touch 512 contiguous bytes.  (Forward fragments read from L1
-// and L2 one layer ahead instead, 42 KB a wave and chunk, took 72 us where this takes 67.)
+// and L2 one layer ahead instead, 42 KB a wave and chunk, took 5 us longer.)
 // Bound by LDS: about 1.1 MB a chunk of both rows (fragments, activations, dW operands), then
-// the chain's latency.  293 rows of 8 chunks (16 caches): 85.2 -> 67 us.
+// the chain's latency.  288 rows of 8 chunks (16 caches): 85 -> 69 us.
 template <int H> struct DualGradSmem {
 	_Float16 w[(H * 8 + 2) * 512]; // forward A fragments: [block][run][16 g + r][4]
 	struct Row {
